@@ -158,10 +158,10 @@ double scs_graph_core_time_us(const scs_graph* g);
  * already in device memory (d_off: n+1 int64, d_adj: int32, both device
  * pointers, a simple symmetric graph), written to d_core (n words, device),
  * on `stream` (a hipStream_t; NULL = the default stream).  Working memory is
- * a fixed device array inside the library (3 * 2^20 + 64 words, 12 MB per
+ * a fixed device array inside the library (2 * 2^20 + 1024 words, 8 MB per
  * GPU, held until the process ends), so n is at most 2^20 (SCS_EBIG beyond).
- * Allocates nothing.  Every call on one GPU uses that GPU's array: calls
- * that overlap on one GPU race. */
+ * Allocates nothing.  Every call on one GPU uses that GPU's array: calls of
+ * one process take turns, calls of several threads included. */
 #define SCS_CORE_NOALLOC_MAX_N (1u << 20)
 int scs_core_numbers_noalloc(const int64_t* d_off, const int32_t* d_adj, uint32_t n,
                              uint32_t* d_core, void* stream);

@@ -24,11 +24,9 @@
 void scs_pack_model(const scs_model* m, MlpDev* d);
 
 extern "C" {
-hipError_t scs_launch_core_init(const i64* off, u32 n, u32* deg, u32* core, hipStream_t s);
-hipError_t scs_launch_core_scan(u32 n, u32 k, const u32* deg, u32* core, u32* F, u32* fcount,
-                                u32* minrest, hipStream_t s);
-hipError_t scs_launch_core_peel(const i64* off, const int32_t* adj, u32 k, const u32* F, u32 fn,
-                                u32* deg, u32* core, u32* Fn, u32* fncount, hipStream_t s);
+int scs_core_run(const i64* off, const int32_t* adj, u32 n, u32* core, u32* tmp,
+                 hipStream_t s);
+u64 scs_core_words(u32 n);
 hipError_t scs_launch_ms_init(u32 n, const u32* core, const MsBatch* B, u64* elig, u64* vis,
                               u64* fr, u64* nf, u32* flags, u32 nflags, unsigned long long* bytes,
                               hipStream_t s);
@@ -106,61 +104,26 @@ static int core_decompose(scs_graph* G) {
   const u32 n = G->hg.n;
   hipStream_t s;
   HIPCHK(hipStreamCreate(&s));
-  u32 *deg, *F, *Fn, *cnt;
-  HIPCHK(hipMalloc(&deg, sizeof(u32) * std::max<u32>(n, 1)));
-  HIPCHK(hipMalloc(&F, sizeof(u32) * std::max<u32>(n, 1)));
-  HIPCHK(hipMalloc(&Fn, sizeof(u32) * std::max<u32>(n, 1)));
-  HIPCHK(hipMalloc(&cnt, sizeof(u32) * 4));
-  u32* h_cnt;
-  HIPCHK(hipHostMalloc(&h_cnt, sizeof(u32) * 4));
+  u32* tmp;
+  HIPCHK(hipMalloc(&tmp, sizeof(u32) * scs_core_words(n)));
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
   HIPCHK(hipEventRecord(e0, s));
-  HIPCHK(scs_launch_core_init(G->d_off, n, deg, G->d_core, s));
-  u32 peeled = 0, k = 0;
-  while (peeled < n) {
-    // cnt[0] = frontier size, cnt[1] = min remaining degree
-    u32 init[2] = {0, 0xffffffffu};
-    HIPCHK(hipMemcpyAsync(cnt, init, sizeof(init), hipMemcpyHostToDevice, s));
-    HIPCHK(scs_launch_core_scan(n, k, deg, G->d_core, F, cnt, cnt + 1, s));
-    HIPCHK(hipMemcpyAsync(h_cnt, cnt, 2 * sizeof(u32), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-    u32 fn = h_cnt[0], minrest = h_cnt[1];
-    if (fn == 0) {
-      if (minrest == 0xffffffffu) break;
-      k = std::max(k + 1, minrest);
-      continue;
-    }
-    peeled += fn;
-    u32 *cur = F, *nxt = Fn;
-    while (fn) {
-      HIPCHK(hipMemsetAsync(cnt + 2, 0, sizeof(u32), s));
-      HIPCHK(scs_launch_core_peel(G->d_off, G->d_adj, k, cur, fn, deg, G->d_core, nxt, cnt + 2, s));
-      HIPCHK(hipMemcpyAsync(h_cnt + 2, cnt + 2, sizeof(u32), hipMemcpyDeviceToHost, s));
-      HIPCHK(hipStreamSynchronize(s));
-      fn = h_cnt[2];
-      peeled += fn;
-      std::swap(cur, nxt);
-    }
-    k++;
-  }
+  const int rc = scs_core_run(G->d_off, G->d_adj, n, G->d_core, tmp, s);
   HIPCHK(hipEventRecord(e1, s));
   HIPCHK(hipEventSynchronize(e1));
   float ms = 0;
   HIPCHK(hipEventElapsedTime(&ms, e0, e1));
   G->core_us = ms * 1000.0;
   G->hg.core.resize(n);
-  HIPCHK(hipMemcpy(G->hg.core.data(), G->d_core, sizeof(u32) * n, hipMemcpyDeviceToHost));
-  HIPCHK(hipFree(deg));
-  HIPCHK(hipFree(F));
-  HIPCHK(hipFree(Fn));
-  HIPCHK(hipFree(cnt));
-  HIPCHK(hipHostFree(h_cnt));
+  if (!rc)
+    HIPCHK(hipMemcpy(G->hg.core.data(), G->d_core, sizeof(u32) * n, hipMemcpyDeviceToHost));
+  HIPCHK(hipFree(tmp));
   HIPCHK(hipEventDestroy(e0));
   HIPCHK(hipEventDestroy(e1));
   HIPCHK(hipStreamDestroy(s));
-  return SCS_OK;
+  return rc;
 }
 
 static int graph_upload(scs_graph* G) {

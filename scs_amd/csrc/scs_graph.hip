@@ -6,114 +6,405 @@
 
 #include <mutex>
 
-#define BLK 256
+// ---------------------------------------------------------------------------
+// Core decomposition: level-synchronous peeling in one persistent kernel.
+// deg holds the remaining degree of a live vertex and, once it is peeled, its
+// core number, so the output array is the only n-sized state that changes.
+// At level k every block takes the vertices of its share with deg == k into
+// its LDS queue, a grid barrier ends the scan, and each block then empties
+// its queue: a neighbour whose degree falls to k joins the queue of the block
+// that took it there, so a cascade inside a level needs no further barrier.
+// Entries that do not fit the queue go to a list in device memory, which all
+// blocks share out after the level's barrier.  Core numbers are unique, so
+// the result equals any exact sequential peeling.
+//
+// Bound: latency.  A level costs two grid barriers (4 us each), a scan (10 us)
+// and its longest cascade (queue, offsets, neighbours, degree atomics: 4 us a
+// step); the innermost core, thousands of hubs that leave together, is bound
+// by atomics on the same degrees (2 ms).  Chung-Lu graphs, 88K / 1.5M / 8M
+// edges (16 / 76 / 206 levels): 0.47 / 1.9 / 7.0 ms, 3.0 / 17.0 / 40.7 ms
+// before, with a launch and a host round trip per cascade step.  Blocks of
+// 256 and 1,024 threads are 2-12 % slower on these three, 2,048 vertices per
+// block and more 1.5 times slower on the first.
+// ---------------------------------------------------------------------------
+#define CORE_T 512          // threads per block
+#define CORE_QCAP 4096      // LDS queue entries per block
+#define CORE_EMPTY 0xffffffffu
+#define CORE_VPB 256        // vertices per block at least
+#define CORE_TIMEOUT 3000000000ull  // wall_clock64 ticks (100 MHz): 30 s
 
-// ---------------------------------------------------------------------------
-// Core decomposition: level-synchronous peeling.  At level k the vertices
-// still alive with degree <= k are peeled (core = k); every decrement that
-// takes a neighbour from k+1 to k appends it to the next frontier of the
-// same level.  Core numbers are unique, so the result equals any exact
-// sequential peeling.
-// ---------------------------------------------------------------------------
-__global__ void core_init(const i64* __restrict__ off, u32 n, u32* __restrict__ deg,
-                          u32* __restrict__ core) {
-  for (u32 v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
-    deg[v] = (u32)(off[v + 1] - off[v]);
-    core[v] = 0xffffffffu;
+enum { CORE_SCAN = 0, CORE_PEEL = 1, CORE_OVF = 2, CORE_DONE = 3 };
+
+// Barrier and counters, 128-byte lines apart (a line that others poll makes
+// an atomic on it wait).  Blocks arrive in CORE_GROUPS groups (by block
+// number, which is how blocks are dealt to the XCDs), the last of a group
+// arrives at the root: 32 + 8 serial adds instead of 256.  An arrival adds
+// one in the low word and its count of vertices in the high word.
+#define CORE_GROUPS 8
+struct __attribute__((aligned(128))) CoreLine {
+  u64 v;
+  u64 pad[15];
+};
+struct CoreCtl {
+  CoreLine grp[CORE_GROUPS];
+  CoreLine go[CORE_GROUPS];  // what the group polls: step << 34 | op << 32 | k
+  CoreLine root;
+  u32 minrest, pad0[31];
+  u32 ovf, pad1[31];
+  // the root's last block only
+  u32 k, o0, o1, peeled, failed;
+};
+#define CORE_CTL_WORDS 1024
+static_assert(sizeof(CoreCtl) <= CORE_CTL_WORDS * sizeof(u32), "fits the counter words");
+
+__device__ __forceinline__ u32 c_load(const u32* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void c_store(u32* p, u32 v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Place of vertex v's degree: an odd multiple modulo the power of two above
+// n.  Generators and crawls number hubs first, and 32 hubs' degrees in one
+// cache line make every decrement of any of them wait for the others.
+#define CORE_MUL 0x9E3779B1u
+#define CORE_INV 0x0E8B2F51u
+__device__ __forceinline__ u32 core_pos(u32 v, u32 mask) { return (v * CORE_MUL) & mask; }
+
+__global__ void core_init(const i64* __restrict__ off, u32 n, u32* __restrict__ deg, u32 mask,
+                          CoreCtl* __restrict__ ctl) {
+  for (u32 v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
+    deg[core_pos(v, mask)] = (u32)(off[v + 1] - off[v]);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    CoreCtl c{};
+    c.minrest = 0xffffffffu;
+    *ctl = c;  // one thread: a few hundred words, once per run
   }
 }
 
-// Appends alive vertices with deg <= k to F (sets core = k) and computes the
-// minimum degree among the remaining alive vertices.
-__global__ void core_scan(u32 n, u32 k, const u32* __restrict__ deg, u32* __restrict__ core,
-                          u32* __restrict__ F, u32* __restrict__ fcount, u32* __restrict__ minrest) {
-  u32 mn = 0xffffffffu;
-  for (u32 v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
-    if (core[v] != 0xffffffffu) continue;
-    u32 d = deg[v];
-    if (d <= k) {
-      core[v] = k;
-      F[atomicAdd(fcount, 1u)] = v;
-    } else {
-      mn = min(mn, d);
-    }
-  }
-  for (int o = 32; o > 0; o >>= 1) mn = min(mn, (u32)__shfl_xor((int)mn, o));
-  if ((threadIdx.x & 63) == 0 && mn != 0xffffffffu) atomicMin(minrest, mn);
+struct CoreLds {
+  u32 q[CORE_QCAP];
+  u32 head, tail, pending, done;
+  u32 found, op, k, o0, o1, mn;
+};
+__device__ __forceinline__ u32 c_lget(const u32* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void c_lput(u32* p, u32 v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// One wave per frontier vertex; decrements alive neighbours.
-__global__ void core_peel(const i64* __restrict__ off, const int32_t* __restrict__ adj, u32 k,
-                          const u32* __restrict__ F, u32 fn, u32* __restrict__ deg,
-                          u32* __restrict__ core, u32* __restrict__ Fn, u32* __restrict__ fncount) {
-  const u32 lane = threadIdx.x & 63;
-  const u32 wid = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const u32 nw = (gridDim.x * blockDim.x) >> 6;
-  for (u32 i = wid; i < fn; i += nw) {
-    u32 v = F[i];
-    i64 b = off[v], e = off[v + 1];
-    for (i64 j = b + lane; j < e; j += 64) {
-      u32 w = (u32)adj[j];
-      if (core[w] != 0xffffffffu) continue;
-      u32 old = atomicSub(&deg[w], 1u);
-      if (old == k + 1) {
-        core[w] = k;
-        Fn[atomicAdd(fncount, 1u)] = w;
+__device__ __forceinline__ u64 c_add64(u64* p, u64 v) {
+  return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void c_store64(u64* p, u64 v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Everything blocks exchange goes through agent-scope atomic loads, stores
+// and adds, which act at the memory all XCDs share.  What one block must see
+// after another is ordered by waiting for those operations alone: a release
+// or acquire at agent scope would also write back the XCD's L2 or drop its
+// lines, once per block and barrier (8 us of a 12 us step here).
+__device__ __forceinline__ void c_order() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+  __builtin_amdgcn_s_waitcnt(0);
+}
+__device__ __forceinline__ u64 c_load64(const u64* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Grid barrier after step `gen`; the last block to arrive decides the next
+// step for all.  scan: the barrier ends a scan that queued `count` vertices,
+// else a peel that finished `count`.  The step comes back in L.
+__device__ void core_barrier(CoreCtl* C, CoreLds& L, u32 n, u32 gen, bool scan, u32 count) {
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const u32 g = blockIdx.x % CORE_GROUPS, G = gridDim.x;
+    const u32 ingrp = (G - g + CORE_GROUPS - 1) / CORE_GROUPS;
+    const u32 ngrp = G < CORE_GROUPS ? G : CORE_GROUPS;
+    if (scan && L.mn < c_load(&C->minrest)) atomicMin(&C->minrest, L.mn);
+    c_order();
+    const u64 mine = ((u64)count << 32) | 1ull;
+    const u64 a = c_add64(&C->grp[g].v, mine) + mine;
+    if ((u32)a == ingrp) {
+      c_store64(&C->grp[g].v, 0ull);
+      c_order();
+      const u64 gm = (a & 0xFFFFFFFF00000000ull) | 1ull;
+      const u64 r = c_add64(&C->root.v, gm) + gm;
+      if ((u32)r == ngrp) {
+        const u32 total = (u32)(r >> 32), k = c_load(&C->k);
+        u32 op, nk = k;
+        if (scan) {
+          const u32 mr = c_load(&C->minrest);
+          if (total) {
+            op = CORE_PEEL;
+          } else if (mr == 0xffffffffu) {
+            op = CORE_DONE;
+          } else {
+            op = CORE_SCAN;
+            nk = mr > k + 1 ? mr : k + 1;
+          }
+          c_store(&C->minrest, 0xffffffffu);
+        } else {
+          const u32 ov = c_load(&C->ovf), o1 = c_load(&C->o1), pe = c_load(&C->peeled) + total;
+          c_store(&C->peeled, pe);
+          if (ov > o1) {
+            op = CORE_OVF;
+            c_store(&C->o0, o1);
+            c_store(&C->o1, ov);
+          } else {
+            op = pe >= n ? CORE_DONE : CORE_SCAN;
+            nk = k + 1;
+          }
+        }
+        c_store(&C->k, nk);
+        c_store64(&C->root.v, 0ull);
+        c_order();
+        const u64 w = ((u64)(gen + 1) << 34) | ((u64)op << 32) | nk;
+        for (u32 i = 0; i < ngrp; i++) c_store64(&C->go[i].v, w);
       }
     }
+    // every block of the grid is resident, so the wait ends; the time limit
+    // only guards against a machine where that does not hold
+    u64 w;
+    const u64 t0 = wall_clock64();
+    u32 spins = 0;
+    bool bad = false;
+    while ((u32)((w = c_load64(&C->go[g].v)) >> 34) != gen + 1) {
+      __builtin_amdgcn_s_sleep(1);
+      if ((++spins & 1023u) == 0 &&
+          (c_load(&C->failed) || wall_clock64() - t0 > CORE_TIMEOUT)) {
+        c_store(&C->failed, 1u);
+        bad = true;
+        break;
+      }
+    }
+    c_order();
+    L.op = bad ? (u32)CORE_DONE : (u32)(w >> 32) & 3u;
+    L.k = (u32)w;
+    if (L.op == CORE_OVF) {
+      L.o0 = c_load(&C->o0);
+      L.o1 = c_load(&C->o1);
+    }
   }
+  __syncthreads();
+}
+
+__device__ __forceinline__ void core_push(CoreCtl* C, CoreLds& L, u32* ovf, u32 v) {
+  const u32 p = atomicAdd(&L.tail, 1u);
+  if (p < CORE_QCAP) {
+    atomicAdd(&L.pending, 1u);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    c_lput(&L.q[p], v);
+  } else {
+    c_store(&ovf[atomicAdd(&C->ovf, 1u)], v);
+  }
+}
+
+// Peels v with one wave, four adjacency entries per lane in flight (the next
+// four are loaded before this step's degree atomics).  Takes one from each
+// live neighbour's degree; the lane that takes it to k queues the neighbour,
+// and a decrement that lost the race against that one is undone.  Looking at
+// the degree first costs a round trip per step of a cascade (4,000 vertices:
+// 480 us, 370 without) and saves two atomics per peeled neighbour (500,000
+// vertices: 7.2 ms, 12.7 without).
+__device__ __forceinline__ void core_take(const i64* __restrict__ off,
+                                          const int32_t* __restrict__ adj, CoreCtl* C, CoreLds& L,
+                                          u32* ovf, u32* deg, u32 mask, u32 k, u32 v) {
+  const u32 lane = threadIdx.x & 63;
+  const i64 b = off[v], e = off[v + 1];
+  if (b == e) return;
+  u32 w[4], x[4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) w[t] = b + lane + 64 * t < e ? (u32)adj[b + lane + 64 * t] : v;
+  for (i64 j = b + lane; j - (i64)lane < e; j += 256) {
+#pragma unroll
+    for (int t = 0; t < 4; t++) x[t] = j + 256 + 64 * t < e ? (u32)adj[j + 256 + 64 * t] : v;
+    u32 old[4];
+    u32 d[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) d[t] = c_load(&deg[core_pos(w[t], mask)]);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+      old[t] = w[t] != v && d[t] > k ? atomicSub(&deg[core_pos(w[t], mask)], 1u) : 0xffffffffu;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      if (old[t] == k + 1)
+        core_push(C, L, ovf, w[t]);
+      else if (old[t] <= k)
+        atomicAdd(&deg[core_pos(w[t], mask)], 1u);
+      w[t] = x[t];
+    }
+  }
+}
+
+__global__ void __launch_bounds__(CORE_T) core_peel(const i64* __restrict__ off,
+                                                    const int32_t* __restrict__ adj, u32 n,
+                                                    u32* __restrict__ core, u32* __restrict__ deg,
+                                                    u32 mask, u32* __restrict__ ovf,
+                                                    CoreCtl* __restrict__ C) {
+  __shared__ CoreLds L;
+  const u32 nt = gridDim.x * CORE_T, tid = blockIdx.x * CORE_T + threadIdx.x;
+  const u32 lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (u32 i = threadIdx.x; i < CORE_QCAP; i += CORE_T) L.q[i] = CORE_EMPTY;
+  if (threadIdx.x == 0) {
+    L.tail = L.head = L.pending = L.done = 0;
+    L.op = CORE_SCAN;
+    L.k = 0;
+  }
+  __syncthreads();
+  // each pass of the loop ends in one grid barrier
+  for (u32 gen = 0;; gen++) {
+    const u32 op = L.op, k = L.k, o0 = L.o0, o1 = L.o1;
+    if (op == CORE_DONE) break;
+    if (op == CORE_SCAN) {
+      if (threadIdx.x == 0) {
+        L.found = 0;
+        L.mn = 0xffffffffu;
+      }
+      __syncthreads();
+      u32 mn = 0xffffffffu, fnd = 0;
+      for (u64 p0 = tid; p0 <= mask; p0 += 4ull * nt) {
+        u32 d[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          const u64 p = p0 + (u64)t * nt;
+          d[t] = p <= mask ? c_load(&deg[p]) : 0u;
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          const u64 p = p0 + (u64)t * nt;
+          const u32 v = ((u32)p * CORE_INV) & mask;
+          if (p > mask || v >= n) continue;
+          if (d[t] == k) {
+            core_push(C, L, ovf, v);
+            fnd++;
+          } else if (d[t] > k) {
+            mn = min(mn, d[t]);
+          }
+        }
+      }
+      for (int o = 32; o > 0; o >>= 1) {
+        mn = min(mn, (u32)__shfl_xor((int)mn, o));
+        fnd += (u32)__shfl_xor((int)fnd, o);
+      }
+      if ((threadIdx.x & 63) == 0) {
+        if (fnd) atomicAdd(&L.found, fnd);
+        atomicMin(&L.mn, mn);
+      }
+      __syncthreads();
+      core_barrier(C, L, n, gen, true, L.found);
+      continue;
+    }
+    u32 done = 0;
+    if (op == CORE_OVF) {
+      // this block's share of the entries that overflowed, a wave each
+      for (u64 i = (u64)wave * gridDim.x + blockIdx.x; i < o1 - o0;
+           i += (u64)gridDim.x * (CORE_T / 64)) {
+        core_take(off, adj, C, L, ovf, deg, mask, k, c_load(&ovf[o0 + i]));
+        done++;
+      }
+    }
+    // This block's queue, until its cascades end: a wave holds one ticket
+    // (queue position) at a time, waits for its entry, and leaves when the
+    // queue has no entry for it and none is being peeled (pending counts
+    // entries queued and not yet peeled, so a wave that may still queue
+    // others keeps it above zero).
+    if (op == CORE_OVF) __syncthreads();
+    while (true) {
+      u32 h = 0, v = CORE_EMPTY;
+      if (lane == 0) {
+        h = atomicAdd(&L.head, 1u);
+        if (h < CORE_QCAP) {
+          while (true) {
+            v = c_lget(&L.q[h]);
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            if (v != CORE_EMPTY || c_lget(&L.pending) == 0) break;
+            __builtin_amdgcn_s_sleep(1);
+          }
+        }
+      }
+      v = __builtin_amdgcn_readfirstlane(v);
+      if (v == CORE_EMPTY) break;
+      core_take(off, adj, C, L, ovf, deg, mask, k, v);
+      done++;
+      // after this wave's pushes: a wave's LDS operations are done in order
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      if (lane == 0) atomicSub(&L.pending, 1u);
+    }
+    __syncthreads();
+    for (u32 i = threadIdx.x; i < min(L.tail, (u32)CORE_QCAP); i += CORE_T) L.q[i] = CORE_EMPTY;
+    if (lane == 0 && done) atomicAdd(&L.done, done);
+    __syncthreads();
+    done = L.done;
+    __syncthreads();
+    if (threadIdx.x == 0) L.tail = L.head = L.done = 0;
+    core_barrier(C, L, n, gen, false, done);
+  }
+  for (u32 v = tid; v < n; v += nt) core[v] = c_load(&deg[core_pos(v, mask)]);
 }
 
 // ---------------------------------------------------------------------------
 // Host-side launch helpers (C linkage inside the library).
 // ---------------------------------------------------------------------------
-static inline u32 nblocks(u64 work, u32 per, u32 cap) {
-  u64 b = (work + per - 1) / per;
-  if (b < 1) b = 1;
-  if (b > cap) b = cap;
-  return (u32)b;
+// One block per CU at most (every block must be resident for the grid
+// barrier: 8 waves and 17 KB of LDS), fewer on small graphs, whose levels
+// are too short for every CU to have a share.
+static u32 core_blocks(u32 n) {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      cus < 1)
+    cus = 1;
+  const u32 want = n / CORE_VPB + 1;
+  return want < (u32)cus ? want : (u32)cus;
 }
 
-extern "C" hipError_t scs_launch_core_init(const i64* off, u32 n, u32* deg, u32* core,
-                                           hipStream_t s) {
-  core_init<<<nblocks(n, BLK, 4096), BLK, 0, s>>>(off, n, deg, core);
-  return hipGetLastError();
+static u32 core_pow2(u32 n) {
+  u32 b = 0;
+  while ((1ull << b) < n) b++;
+  return b;
 }
-extern "C" hipError_t scs_launch_core_scan(u32 n, u32 k, const u32* deg, u32* core, u32* F,
-                                           u32* fcount, u32* minrest, hipStream_t s) {
-  core_scan<<<nblocks(n, BLK, 4096), BLK, 0, s>>>(n, k, deg, core, F, fcount, minrest);
-  return hipGetLastError();
-}
-extern "C" hipError_t scs_launch_core_peel(const i64* off, const int32_t* adj, u32 k, const u32* F,
-                                           u32 fn, u32* deg, u32* core, u32* Fn, u32* fncount,
-                                           hipStream_t s) {
-  core_peel<<<nblocks((u64)fn * 64, BLK, 8192), BLK, 0, s>>>(off, adj, k, F, fn, deg, core, Fn,
-                                                             fncount);
-  return hipGetLastError();
+// Words of scs_core_run's working memory: counters, degrees, overflow list.
+extern "C" u64 scs_core_words(u32 n) { return CORE_CTL_WORDS + (1ull << core_pow2(n)) + n; }
+
+// Core numbers of the CSR into core; tmp: scs_core_words(n) words on a
+// 128-byte boundary.  One peel runs on a device at a time: two grids that
+// each wait for all their blocks must not share it.  Waits for the result.
+static std::mutex g_core_mu;
+extern "C" int scs_core_run(const i64* off, const int32_t* adj, u32 n, u32* core, u32* tmp,
+                            hipStream_t s) {
+  if (n == 0) return SCS_OK;
+  std::lock_guard<std::mutex> lk(g_core_mu);
+  CoreCtl* C = (CoreCtl*)tmp;
+  const u64 slots = 1ull << core_pow2(n);
+  u32* deg = tmp + CORE_CTL_WORDS;
+  u32* ovf = deg + slots;
+  const u32 ib = (n + 255) / 256;
+  core_init<<<ib < 4096 ? ib : 4096, 256, 0, s>>>(off, n, deg, (u32)(slots - 1), C);
+  if (hipGetLastError() != hipSuccess) return SCS_EHIP;
+  core_peel<<<core_blocks(n), CORE_T, 0, s>>>(off, adj, n, core, deg, (u32)(slots - 1), ovf, C);
+  if (hipGetLastError() != hipSuccess) return SCS_EHIP;
+  u32 failed = 0;
+  if (hipMemcpyAsync(&failed, &C->failed, sizeof(u32), hipMemcpyDeviceToHost, s) != hipSuccess ||
+      hipStreamSynchronize(s) != hipSuccess)
+    return SCS_EHIP;
+  return failed ? SCS_EHIP : SCS_OK;
 }
 
 // ---------------------------------------------------------------------------
 // Core numbers without allocation, for callers that cannot allocate device
-// memory.  The working memory (degrees, two frontiers, three counters) is
+// memory.  The working memory (overflow list, barrier and counter words) is
 // this fixed device array; the host finds its per-device address once with
 // hipGetSymbolAddress and passes that address to the kernels.
-// Layout (words): deg[CORE_NA_MAX_N] | F[..] | Fn[..] | counters[64].
+// Layout (words): counters[CORE_CTL_WORDS] | degrees | overflow list.
 // ---------------------------------------------------------------------------
 #define CORE_NA_MAX_N (1u << 20)
-static __device__ __align__(256) u32 scratch[3u * CORE_NA_MAX_N + 64];
+static __device__ __align__(256) u32 scratch[CORE_CTL_WORDS + 2u * CORE_NA_MAX_N];
 
 #define CORE_NA_DEVICES 64
 static u32* g_scratch_dev[CORE_NA_DEVICES];
 static std::mutex g_scratch_mu;
-
-// cnt[0..3) = a, b, c (a kernel, not a memset: callers may capture this)
-__global__ void core_counters(u32* cnt, u32 a, u32 b, u32 c) {
-  if (threadIdx.x == 0) {
-    cnt[0] = a;
-    cnt[1] = b;
-    cnt[2] = c;
-  }
-}
 
 static int scratch_address(u32** out) {
   int dev = 0;
@@ -128,11 +419,6 @@ static int scratch_address(u32** out) {
   return SCS_OK;
 }
 
-#define NA_CHK(x)                          \
-  do {                                     \
-    if ((x) != hipSuccess) return SCS_EHIP; \
-  } while (0)
-
 extern "C" int scs_core_numbers_noalloc(const int64_t* d_off, const int32_t* d_adj, uint32_t n,
                                         uint32_t* d_core, void* stream) {
   if (!d_off || !d_core || (n && !d_adj)) return SCS_EINVAL;
@@ -141,43 +427,5 @@ extern "C" int scs_core_numbers_noalloc(const int64_t* d_off, const int32_t* d_a
   u32* S = nullptr;
   const int rc = scratch_address(&S);
   if (rc) return rc;
-  u32* deg = S;
-  u32* F = S + CORE_NA_MAX_N;
-  u32* Fn = S + 2u * CORE_NA_MAX_N;
-  u32* cnt = S + 3u * CORE_NA_MAX_N;
-  hipStream_t s = (hipStream_t)stream;
-  NA_CHK(scs_launch_core_init(d_off, n, deg, d_core, s));
-  u32 peeled = 0, k = 0;
-  while (peeled < n) {
-    // cnt[0] = frontier size, cnt[1] = min remaining degree
-    core_counters<<<1, 64, 0, s>>>(cnt, 0u, 0xffffffffu, 0u);
-    NA_CHK(hipGetLastError());
-    NA_CHK(scs_launch_core_scan(n, k, deg, d_core, F, cnt, cnt + 1, s));
-    u32 h[2];
-    NA_CHK(hipMemcpyAsync(h, cnt, sizeof(h), hipMemcpyDeviceToHost, s));
-    NA_CHK(hipStreamSynchronize(s));
-    u32 fn = h[0];
-    if (fn == 0) {
-      if (h[1] == 0xffffffffu) break;
-      k = h[1] > k + 1 ? h[1] : k + 1;
-      continue;
-    }
-    peeled += fn;
-    u32 *cur = F, *nxt = Fn;
-    while (fn) {
-      core_counters<<<1, 64, 0, s>>>(cnt, 0u, 0xffffffffu, 0u);
-      NA_CHK(hipGetLastError());
-      NA_CHK(scs_launch_core_peel(d_off, d_adj, k, cur, fn, deg, d_core, nxt, cnt + 2, s));
-      u32 f2 = 0;
-      NA_CHK(hipMemcpyAsync(&f2, cnt + 2, sizeof(u32), hipMemcpyDeviceToHost, s));
-      NA_CHK(hipStreamSynchronize(s));
-      fn = f2;
-      peeled += fn;
-      u32* t = cur;
-      cur = nxt;
-      nxt = t;
-    }
-    k++;
-  }
-  return SCS_OK;
+  return scs_core_run(d_off, d_adj, n, d_core, S, (hipStream_t)stream);
 }
