@@ -108,9 +108,9 @@ struct Lds {
   u32 D[SCS_FRAME_DOMS];
   u32 hist[SCS_HCAP + 4];   // dC histogram of R (live copy of the wave's state)
   u64 tot[64];              // per-vertex sums of a scan_adj step
-  union {                   // never live at the same time within a node
+  union __attribute__((aligned(8))) {  // never live at the same time within a node
     u32 chist[SCS_HCAP + 4];  // scratch histogram of C degrees (U_nr)
-    u16 h1s[16 * MLP_H];      // MLP hidden-layer tile (bf16)
+    u16 h1s[16 * MLP_H];      // MLP hidden-layer tile (bf16), 8-byte aligned
   };
 };
 
@@ -1226,6 +1226,7 @@ __device__ __forceinline__ MlpFeat cand_features(const W& w, u32 x, u32 Cs, u32 
 __device__ __forceinline__ u32 learned_ustar(W& w, const u32* cand, u32 nf, u32 Cs, u32 kl) {
   float bestf = -INFINITY;
   u32 bestx = INV;
+  const MlpMem R(w.model);
 #pragma unroll 1
   for (u32 t0 = 0; t0 < nf; t0 += 16) {
     auto feat = [&](u32 row) {
@@ -1233,7 +1234,7 @@ __device__ __forceinline__ u32 learned_ustar(W& w, const u32* cand, u32 nf, u32 
       if (i < nf) return cand_features(w, cand[i], Cs, kl);
       return MlpFeat{0, 0, 0, 0, 0, 0.f};
     };
-    const float sc = mlp_tile(w.model, feat, w.L->h1s);
+    const float sc = mlp_tile(R, feat, w.L->h1s);
     const u32 i = t0 + (LANE & 15u);
     if (LANE < 16 && i < nf) {
       const u32 x = cand[i];

@@ -23,8 +23,10 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 // Packed inference model in device memory.
 struct MlpDev {
-  u16 w1[MLP_INP][MLP_H];  // bf16, rows >= MLP_IN are zero
-  u16 w2[MLP_H][MLP_H];    // bf16
+  // bf16, [output unit][input]: a lane's four inputs of an MFMA step are one
+  // 8-byte load
+  u16 w1[MLP_H][MLP_INP];  // inputs >= MLP_IN are zero
+  u16 w2[MLP_H][MLP_H];
   float b1[MLP_H];
   float b2[MLP_H];
   float w3[MLP_H];
@@ -49,71 +51,113 @@ struct MlpFeat {
   float cscore;
 };
 
+// The model as mlp_tile takes it.  MlpRegs: the wave's share in registers,
+// loaded once and used for many tiles (stand-alone inference; 60 registers).
+// MlpMem: read again for every tile, one group of 16 units at a time (the
+// search kernel, whose own state leaves no room: held in registers there the
+// model spilled 396 bytes per lane).
+struct MlpMem {
+  static constexpr int UNROLL = 1;
+  const MlpDev* M;
+  u32 row, kb;
+  __device__ explicit MlpMem(const MlpDev* m)
+      : M(m), row(threadIdx.x & 15u), kb((threadIdx.x & 63u) >> 4) {}
+  __device__ bf16x4 w1(u32 j) const { return *(const bf16x4*)&M->w1[16 * j + row][4 * kb]; }
+  __device__ bf16x4 w2(u32 j, u32 ks) const {
+    return *(const bf16x4*)&M->w2[16 * j + row][16 * ks + 4 * kb];
+  }
+  __device__ float b1(u32 j) const { return M->b1[16 * j + row]; }
+  __device__ float b2(u32 j) const { return M->b2[16 * j + row]; }
+  __device__ float w3(u32 j) const { return M->w3[16 * j + row]; }
+  __device__ float b3() const { return M->b3; }
+  // of this lane's input 4*kb + i (0 beyond the sixth)
+  __device__ float mean(u32 i) const { return 4 * kb + i < MLP_IN ? M->mean[4 * kb + i] : 0.f; }
+  __device__ float scale(u32 i) const { return 4 * kb + i < MLP_IN ? M->scale[4 * kb + i] : 0.f; }
+};
+struct MlpRegs {
+  static constexpr int UNROLL = 4;
+  bf16x4 w1_[4], w2_[4][4];
+  float b1_[4], b2_[4], w3_[4], b3_, mean_[4], scale_[4];
+  __device__ explicit MlpRegs(const MlpMem& m) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      w1_[j] = m.w1(j);
+#pragma unroll
+      for (int ks = 0; ks < 4; ks++) w2_[j][ks] = m.w2(j, ks);
+      b1_[j] = m.b1(j);
+      b2_[j] = m.b2(j);
+      w3_[j] = m.w3(j);
+      mean_[j] = m.mean(j);
+      scale_[j] = m.scale(j);
+    }
+    b3_ = m.b3();
+  }
+  __device__ bf16x4 w1(u32 j) const { return w1_[j]; }
+  __device__ bf16x4 w2(u32 j, u32 ks) const { return w2_[j][ks]; }
+  __device__ float b1(u32 j) const { return b1_[j]; }
+  __device__ float b2(u32 j) const { return b2_[j]; }
+  __device__ float w3(u32 j) const { return w3_[j]; }
+  __device__ float b3() const { return b3_; }
+  __device__ float mean(u32 i) const { return mean_[i]; }
+  __device__ float scale(u32 i) const { return scale_[i]; }
+};
+
 // Scores the 16 candidates of one tile.  feat(row) gives the raw features
 // of row (rows >= valid are ignored).  h1s: 16 x 64 bf16 LDS scratch.
 // Returns the score of row (l % 16) on every lane (lanes with the same
 // l % 16 hold the same value).
-template <typename FeatFn>
-__device__ float mlp_tile(const MlpDev* M, FeatFn feat, u16* h1s) {
-  const u32 l = threadIdx.x;
+template <typename Model, typename FeatFn>
+__device__ __forceinline__ float mlp_tile(const Model& R, FeatFn feat, u16* h1s) {
+  const u32 l = threadIdx.x & 63u;
   const u32 row = l & 15u;
   const u32 kb = l >> 4;
   // layer 1 input: 16 rows x 16 k (features 0..5, rest zero)
   MlpFeat f = feat(row);
-  float xin[6];
-  xin[0] = (float)f.dC;
-  xin[1] = (float)f.dR;
-  xin[2] = (float)f.dist;
-  xin[3] = (float)f.core;
-  xin[4] = (float)f.slack;
-  xin[5] = f.cscore;
+  float xin[8] = {(float)f.dC, (float)f.dR,    (float)f.dist, (float)f.core,
+                  (float)f.slack, f.cscore, 0.f,          0.f};
   bf16x4 a1;
+#pragma unroll
   for (int i = 0; i < 4; i++) {
-    const u32 k = 4 * kb + i;
-    float x = 0.f;
-    if (k < MLP_IN) x = (xin[k] - M->mean[k]) * M->scale[k];
-    a1[i] = (short)f2bf(x);
+    const float x = kb == 0 ? xin[i] : (kb == 1 ? xin[4 + i] : 0.f);
+    a1[i] = (short)f2bf((x - R.mean(i)) * R.scale(i));
   }
-#pragma unroll 1
+#pragma unroll Model::UNROLL
   for (u32 j = 0; j < 4; j++) {
-    bf16x4 b;
-    for (int i = 0; i < 4; i++) b[i] = (short)M->w1[4 * kb + i][16 * j + row];
+    const float b1 = R.b1(j);
     f32x4 d = {0.f, 0.f, 0.f, 0.f};
-    d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1, b, d, 0, 0, 0);
-    const u32 col = 16 * j + row;
-    const float bias = M->b1[col];
+    d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1, R.w1(j), d, 0, 0, 0);
+#pragma unroll
     for (int i = 0; i < 4; i++) {
-      float z = d[i] + bias;
-      h1s[(4 * kb + i) * MLP_H + col] = f2bf(z > 0.f ? z : 0.f);
+      float z = d[i] + b1;
+      h1s[(4 * kb + i) * MLP_H + 16 * j + row] = f2bf(z > 0.f ? z : 0.f);
     }
   }
   __syncthreads();
   // layer 2 (K = 64 in four steps) fused with the 64 -> 1 output layer
+  bf16x4 a[4];
+#pragma unroll
+  for (u32 ks = 0; ks < 4; ks++) a[ks] = *(const bf16x4*)&h1s[row * MLP_H + 16 * ks + 4 * kb];
   float part[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
+#pragma unroll Model::UNROLL
   for (u32 j = 0; j < 4; j++) {
+    bf16x4 wj[4];
+#pragma unroll
+    for (u32 ks = 0; ks < 4; ks++) wj[ks] = R.w2(j, ks);
+    const float b2 = R.b2(j), w3 = R.w3(j);
     f32x4 d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (u32 ks = 0; ks < 4; ks++) {
-      bf16x4 a, b;
-      for (int i = 0; i < 4; i++) {
-        a[i] = (short)h1s[row * MLP_H + 16 * ks + 4 * kb + i];
-        b[i] = (short)M->w2[16 * ks + 4 * kb + i][16 * j + row];
-      }
-      d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, d, 0, 0, 0);
-    }
-    const u32 col = 16 * j + row;
-    const float bias = M->b2[col], w = M->w3[col];
+#pragma unroll
+    for (u32 ks = 0; ks < 4; ks++)
+      d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[ks], wj[ks], d, 0, 0, 0);
+#pragma unroll
     for (int i = 0; i < 4; i++) {
-      float z = d[i] + bias;
-      part[i] += (z > 0.f ? z : 0.f) * w;
+      float z = d[i] + b2;
+      part[i] += (z > 0.f ? z : 0.f) * w3;
     }
   }
   // part[i] is row (4*kb + i)'s partial sum over this lane's 4 columns;
   // sum over the 16 lanes of the same kb
   for (int i = 0; i < 4; i++)
     for (int o = 8; o > 0; o >>= 1) part[i] += __shfl_xor(part[i], o, 16);
-  // lane l needs row l % 16 = 4*kb' + i'  -> read from a lane of group kb'
   // every lane of group kb now holds the sums of rows 4kb..4kb+3; lane l
   // needs row l % 16, held by group (l % 16) / 4 at index (l % 16) % 4
   const u32 src_kb = row >> 2, src_i = row & 3u;
@@ -121,5 +165,5 @@ __device__ float mlp_tile(const MlpDev* M, FeatFn feat, u16* h1s) {
   const float v2 = __shfl(part[2], 16 * src_kb), v3 = __shfl(part[3], 16 * src_kb);
   const float s = src_i == 0 ? v0 : src_i == 1 ? v1 : src_i == 2 ? v2 : v3;
   __syncthreads();
-  return s + M->b3;
+  return s + R.b3();
 }
