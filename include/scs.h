@@ -118,7 +118,7 @@ typedef struct scs_params {
                               CSR whenever the search state fits; same optimum, node
                               counts and witness in every mode */
   uint32_t gpu_heuristic;  /* 1 = admission computes CSSC_heu (inc/heuristic.h:321-348) on
-                              the GPU, one wave per query, instead of on host threads;
+                              the GPU, three blocks per query, instead of on host threads;
                               same kl and H (needs fewer than 2^32 adjacency entries) */
 } scs_params;
 
@@ -222,7 +222,7 @@ int scs_heuristic_csr(const int64_t* off, const int32_t* adj, uint32_t n, uint32
                       uint32_t* hsize);
 
 /* The same greedy lower bound (inc/heuristic.h:8-348) for `count` queries on
- * the GPU, one wave per construction of each query, on a resident graph: kl[i], hsize[i] (the size
+ * the GPU, one block per construction of each query, on a resident graph: kl[i], hsize[i] (the size
  * of H, also when it exceeds cap) and H row i (up to cap ids).  Equal to
  * scs_heuristic_csr value for value.  SCS_EBIG when the graph has 2^32
  * adjacency entries or more. */

@@ -63,9 +63,9 @@ hipError_t scs_launch_expire(QuerySlot* slots, const u32* idx, u32 n, hipStream_
 hipError_t scs_launch_admit(const EngineArgs* A, const u32* slots, u32 n, u32* failed,
                             hipStream_t s);
 hipError_t scs_launch_pool_init(u64* seq, u32 n, hipStream_t s);
-HeuLayout scs_heu_layout(u32 n, u32 hcap);
+HeuLayout scs_heu_layout(u32 n, u32 hmax);
 hipError_t scs_launch_heu(const u32* off, const u32* adj, u32 n, u32 dmax, u32 nq, const u32* ql,
-                          const u32* qh, const u32* qq, u8* ws, HeuLayout lay, u32 hcap, u32* kl,
+                          const u32* qh, const u32* qq, u8* zs, u8* gs, HeuLayout lay, u32 hcap, u32* kl,
                           u32* hsize, u32* H, u32* kl3, u32* hs3, u32* H3, hipStream_t s);
 }
 
@@ -277,13 +277,15 @@ extern "C" void scs_graph_destroy(scs_graph* g) {
 }
 
 // ---------------------------------------------------------------------------
-// GPU greedy heuristic: up to `waves` queries per launch, three waves each
-// (one per construction), on the graph's 32-bit CSR; the workspace's n-sized
-// arrays start zeroed and every wave leaves its own zeroed again.
+// GPU greedy heuristic: up to `waves` queries per call, three blocks each (one
+// per construction), on the graph's 32-bit CSR; the workspace's n-sized arrays
+// start zeroed and every block leaves its own zeroed again.  A launch takes as
+// many queries as the workspace holds for the call's largest h.
 // ---------------------------------------------------------------------------
 struct HeuGpu {
-  u8* ws = nullptr;
-  HeuLayout lay{};
+  u8 *zs = nullptr, *gs = nullptr;
+  u64 zbytes = 0, gbytes = 0;
+  u32 n = 0;
   u32 waves = 0;
   u32* d_in = nullptr;   // l, h, q (3 * waves)
   u32* d_out = nullptr;  // kl, hsize (2 * waves)
@@ -292,39 +294,63 @@ struct HeuGpu {
   u32* d_H3 = nullptr;    // 3 * waves * SCS_MAX_H
   std::vector<u32> h_out, h_H;
 
-  int init(u32 n, u32 w) {
+  // room for `fit` queries of h <= hmax at once (more of smaller h)
+  int init(u32 n_, u32 w, u32 fit, u32 hmax) {
+    n = n_;
     waves = w;
-    lay = scs_heu_layout(n, SCS_MAX_H);
-    HIPCHK(hipMalloc(&ws, lay.stride * 3 * waves));
-    HIPCHK(hipMemset(ws, 0, lay.stride * 3 * waves));
-    HIPCHK(hipMalloc(&d_in, sizeof(u32) * 3 * waves));
-    HIPCHK(hipMalloc(&d_out, sizeof(u32) * 2 * waves));
-    HIPCHK(hipMalloc(&d_H, sizeof(u32) * (u64)SCS_MAX_H * waves));
-    HIPCHK(hipMalloc(&d_out3, sizeof(u32) * 6 * waves));
-    HIPCHK(hipMalloc(&d_H3, sizeof(u32) * (u64)SCS_MAX_H * 3 * waves));
+    const HeuLayout lay = scs_heu_layout(n, hmax);
+    zbytes = lay.zstride * fit;
+    gbytes = lay.gstride * fit;
+    // one allocation: each one costs its share of a short call
+    const u64 part[7] = {zbytes,
+                         gbytes,
+                         sizeof(u32) * 3 * (u64)waves,
+                         sizeof(u32) * 2 * (u64)waves,
+                         sizeof(u32) * (u64)SCS_MAX_H * waves,
+                         sizeof(u32) * 6 * (u64)waves,
+                         sizeof(u32) * (u64)SCS_MAX_H * 3 * waves};
+    u64 at[7], o = 0;
+    for (int i = 0; i < 7; i++) {
+      at[i] = o;
+      o += (part[i] + 255) & ~255ull;
+    }
+    HIPCHK(hipMalloc(&zs, o));
+    HIPCHK(hipMemset(zs, 0, zbytes));
+    gs = zs + at[1];
+    d_in = (u32*)(zs + at[2]);
+    d_out = (u32*)(zs + at[3]);
+    d_H = (u32*)(zs + at[4]);
+    d_out3 = (u32*)(zs + at[5]);
+    d_H3 = (u32*)(zs + at[6]);
     h_out.resize(2 * waves);
     h_H.resize((size_t)SCS_MAX_H * waves);
     return SCS_OK;
   }
   void release() {
-    for (void* p : {(void*)ws, (void*)d_in, (void*)d_out, (void*)d_H, (void*)d_out3, (void*)d_H3})
-      if (p) (void)hipFree(p);
-    ws = nullptr;
+    if (zs) (void)hipFree(zs);
+    zs = gs = nullptr;
     d_in = d_out = d_H = d_out3 = d_H3 = nullptr;
   }
   // queries i0..i0+cnt (cnt <= waves): kl, and H as vectors
   int run(const scs_graph* g, u32 cnt, const u32* l, const u32* h, const u32* q, u32* kl,
           std::vector<u32>* H, hipStream_t s) {
     std::vector<u32> in(3 * (size_t)cnt);
+    u32 hmax = 1;
     for (u32 i = 0; i < cnt; i++) {
       in[i] = l[i];
       in[cnt + i] = h[i];
       in[2 * cnt + i] = q[i];
+      hmax = std::max(hmax, h[i]);
     }
+    const HeuLayout lay = scs_heu_layout(n, hmax);
+    const u32 fit = (u32)std::min<u64>(cnt, std::min(zbytes / lay.zstride, gbytes / lay.gstride));
+    if (fit == 0) return SCS_ENOMEM;
     HIPCHK(hipMemcpyAsync(d_in, in.data(), sizeof(u32) * 3 * cnt, hipMemcpyHostToDevice, s));
-    HIPCHK(scs_launch_heu(g->d_off32, (const u32*)g->d_adj, g->hg.n, g->hg.dmax, cnt, d_in,
-                          d_in + cnt, d_in + 2 * cnt, ws, lay, SCS_MAX_H, d_out, d_out + cnt, d_H,
-                          d_out3, d_out3 + 3 * cnt, d_H3, s));
+    for (u32 i0 = 0; i0 < cnt; i0 += fit)
+      HIPCHK(scs_launch_heu(g->d_off32, (const u32*)g->d_adj, n, g->hg.dmax,
+                            std::min(fit, cnt - i0), d_in + i0, d_in + cnt + i0,
+                            d_in + 2 * cnt + i0, zs, gs, lay, SCS_MAX_H, d_out + i0, d_out + cnt + i0,
+                            d_H + (u64)i0 * SCS_MAX_H, d_out3, d_out3 + 3 * waves, d_H3, s));
     HIPCHK(hipMemcpyAsync(h_out.data(), d_out, sizeof(u32) * 2 * cnt, hipMemcpyDeviceToHost, s));
     HIPCHK(hipMemcpyAsync(h_H.data(), d_H, sizeof(u32) * (u64)SCS_MAX_H * cnt,
                           hipMemcpyDeviceToHost, s));
@@ -347,7 +373,10 @@ extern "C" int scs_heuristic_gpu(const scs_graph* g, uint32_t count, const uint3
     if (q[i] >= g->hg.n || h[i] == 0 || h[i] > SCS_MAX_H || l[i] > h[i]) return SCS_EINVAL;
   if (count == 0) return SCS_OK;
   HeuGpu hg;
-  int rc = hg.init(g->hg.n, std::min<u32>(count, 64));
+  u32 hmax = 1;
+  for (u32 i = 0; i < count; i++) hmax = std::max(hmax, h[i]);
+  const u32 w = std::min<u32>(count, 64);
+  int rc = hg.init(g->hg.n, w, w, hmax);
   hipStream_t s = nullptr;
   if (rc == SCS_OK && hipStreamCreate(&s) != hipSuccess) rc = SCS_EHIP;
   std::vector<std::vector<u32>> HH(hg.waves);
@@ -668,10 +697,11 @@ extern "C" int scs_engine_create(scs_graph* g, const scs_params* pin, scs_engine
   if (p.gpu_heuristic && g->d_off32) {
     // as many queries per launch as an admission step takes, within 16 GiB
     // of workspace (a launch lasts as long as its slowest query)
-    const u64 stride = 3 * scs_heu_layout(g->hg.n, SCS_MAX_H).stride;
-    const u32 w = (u32)std::max<u64>(16, std::min<u64>(std::max<u32>(p.admit_per_step, 64),
-                                                       (16ull << 30) / std::max<u64>(stride, 1)));
-    if (E->heu_gpu.init(g->hg.n, w) != SCS_OK) return fail(SCS_ENOMEM);
+    const HeuLayout lay = scs_heu_layout(g->hg.n, SCS_MAX_H);
+    const u32 w = std::max<u32>(p.admit_per_step, 64);
+    const u32 fit = (u32)std::min<u64>(w, (16ull << 30) / (lay.zstride + lay.gstride));
+    if (E->heu_gpu.init(g->hg.n, w, std::max<u32>(fit, 16), SCS_MAX_H) != SCS_OK)
+      return fail(SCS_ENOMEM);
   }
   E->st.waves = E->nwaves;
   E->st.kcap = E->kcap;

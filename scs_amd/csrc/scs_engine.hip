@@ -2312,10 +2312,11 @@ __global__ void __launch_bounds__(64, 2) __attribute__((flatten)) scs_epoch(Engi
 }
 
 // Dynamic LDS of one wave: its share of the CU's 160 KB at the requested
-// waves per CU, minus the static part, capped at 48 KB.
+// waves per CU, minus the static part, capped at 48 KB.  2 KB per CU stay free
+// for the heuristic's blocks, which run beside an epoch.
 static u32 epoch_lds_bytes(u32 waves_per_cu) {
   const u32 wpc = waves_per_cu ? waves_per_cu : 16;
-  const i64 share = (i64)(160 * 1024 / wpc) - (i64)sizeof(Lds);
+  const i64 share = (i64)(158 * 1024 / wpc) - (i64)sizeof(Lds);
   i64 b = share < (i64)(48 * 1024) ? share : (i64)(48 * 1024);
   b = b > 0 ? (b & ~(i64)511) : 0;
   return (u32)b;

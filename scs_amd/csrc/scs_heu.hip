@@ -1,11 +1,11 @@
 // Greedy lower bounds on the GPU: the reference's CSSC_heu
 // (inc/heuristic.h:321-348), the best of its three greedy constructions
-// heu2 (:8-120), heu3 (:125-239) and heu4 (:242-317), one wave per
-// construction of each query.
+// heu2 (:8-120), heu3 (:125-239) and heu4 (:242-317), one block of eight
+// waves per construction of each query.
 //
 // The reference drives each construction with a std::priority_queue that
 // holds stale duplicates.  Its pop order reduces to a deterministic choice
-// per step, which a wave makes with a reduction instead of a heap:
+// per step, which a block makes with a reduction instead of a heap:
 //   heu2  add the frontier vertex with the largest (count of H-neighbours,
 //         id); every increment of a count pushes, so the largest pushed key
 //         of a vertex is its current count;
@@ -20,15 +20,29 @@
 // so the doubles are bit-identical.  heu4 drops the reference's +1 on q when
 // q is popped alone (inc/heuristic.h:259), as the host version does.
 //
-// Candidates sit in an append-only list.  Each block of 64 list positions,
-// and each group of 64 blocks, keeps the largest key of its members; keys
-// only rise while a vertex is a candidate, so a rise is an atomic max on its
-// block and group, and only the block and group of the vertex chosen in a
-// step are recomputed.  A step costs the chosen vertex's adjacency plus one
-// pass over the group keys (n / 4096 of them).
+// Candidates sit in an append-only list.  Each block of 64 list positions
+// keeps the largest key of its members; keys only rise while a vertex is a
+// candidate, so a rise is an atomic max on its block, and only the block of
+// the vertex chosen in a step is recomputed.  A step costs the chosen
+// vertex's adjacency, shared by the eight waves, and one pass over the block
+// keys.
+//
+// heu3 keeps, for each vertex, one bit per member of H (in joining order) that
+// it is adjacent to, and H sorted by id with each member's term 1/deg: a score
+// is then a walk over the at most h members, the same for every lane, instead
+// of over the vertex's adjacency.
+//
+// Bound: latency of the steps' dependent loads (offsets, neighbours, their
+// records, the keys): 512 lanes share a chosen hub's thousands of neighbours,
+// four in flight each.  64 queries on a 100,000-vertex, 1.5M-edge power-law
+// graph take 4.8 ms, 108.5 ms with one wave per construction and scores that
+// walked adjacency lists; 8 queries on 4,000 vertices 0.9 and 4.6 ms.
 #include "scs_internal.h"
 
-#define HEU_SMALL 64  // heu3: neighbours of at most this degree are scored by one lane
+#define HEU_T 512     // threads per block
+#define HEU_NW (HEU_T / 64)
+#define HEU_SMALL 32  // heu4: members of at most this degree are counted by one lane
+#define HEU_LDSB 64   // heu4: block keys held in LDS (4,096 members)
 
 struct HeuArgs {
   const u32* off;  // n+1, 32-bit offsets of the resident graph
@@ -37,7 +51,8 @@ struct HeuArgs {
   const u32* ql;
   const u32* qh;
   const u32* qq;
-  u8* ws;
+  u8* zs;  // arrays that are zero between queries
+  u8* gs;  // the others
   HeuLayout lay;
   u32* kl;     // nq
   u32* hsize;  // nq (sizes above hcap are reported, H is cut at hcap)
@@ -48,13 +63,26 @@ struct HeuArgs {
 };
 
 #define LANE (threadIdx.x & 63u)
+#define WAVE (threadIdx.x >> 6)
 
-__device__ __forceinline__ void hsync() { __syncthreads(); }
-// the counters are changed by atomics (performed at the L2), so they are
-// read past the L1
-__device__ __forceinline__ u32 hld(u32* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
+// One vertex's state in a construction.  sta: 0 untouched, 1 candidate (heu4:
+// in S), 2 in H.  cnt: H-neighbours.  deg: degree inside H (heu4: inside S).
+struct __attribute__((aligned(16))) HV {
+  u32 cnt, deg, pos, sta;
+};
+
+// The little LDS a block uses leaves it room beside the search kernel.
+struct HL {
+  u64 wmax[HEU_NW];
+  u32 wmin[HEU_NW];
+  u32 m;        // candidates in the list
+  u32 dv[2];    // H-neighbours of the chosen vertex (by step parity)
+  u32 rank[2];  // members of H with a smaller id (by step parity)
+  u32 best[2];  // heu3: largest id + 1 among the equal keys (by step parity)
+  u32 step, mindeg, remove;
+  u64 bk[HEU_LDSB];
+};
+
 __device__ __forceinline__ u32 h_sum(u32 x) {
   for (int o = 32; o > 0; o >>= 1) x += (u32)__shfl_xor((int)x, o);
   return x;
@@ -63,36 +91,31 @@ __device__ __forceinline__ u32 h_min(u32 x) {
   for (int o = 32; o > 0; o >>= 1) x = min(x, (u32)__shfl_xor((int)x, o));
   return x;
 }
-__device__ __forceinline__ u64 h_shfl64(u64 x, int src) {
-  const u32 lo = (u32)__shfl((int)(u32)x, src), hi = (u32)__shfl((int)(u32)(x >> 32), src);
-  return ((u64)hi << 32) | lo;
-}
 __device__ __forceinline__ u64 h_max64(u64 x) {
   for (int o = 32; o > 0; o >>= 1) {
-    const u64 y = h_shfl64(x, (int)(LANE ^ (u32)o));
+    const u32 lo = (u32)__shfl_xor((int)(u32)x, o), hi = (u32)__shfl_xor((int)(u32)(x >> 32), o);
+    const u64 y = ((u64)hi << 32) | lo;
     x = y > x ? y : x;
   }
   return x;
 }
-__device__ __forceinline__ double h_shfld(double x, int src) {
-  return __longlong_as_double((long long)h_shfl64((u64)__double_as_longlong(x), src));
-}
+__device__ __forceinline__ u64 h_below() { return LANE ? (~0ull >> (64 - LANE)) : 0ull; }
+
 struct HW {
   const u32* off;
   const u32* adj;
-  u32 n, dmax;
-  u8* sta;
-  u8* ins;
-  u32* cnt;
-  u32* deg;
-  double* key;
-  u32* pos;
+  u32 n, dmax, W;
+  HV* hv;
+  u64* key;   // heu3: bits of the largest score pushed, plus one
+  u64* mask;  // heu3: W words per vertex, bit j = adjacent to the j-th member of H
   u32* list;
   u32* rmv;
   u32* th;
-  u64* bkey;  // per block of 64 list positions: the largest member key (0 = none)
-  u64* gkey;  // per group of 64 blocks: the largest block key
-  HeuLds* L;
+  u32* hsort;    // heu3: H sorted by id (two rows of hrow words, by step
+  u32 hrow;      // parity), and each member's joining number (two more rows)
+  double* term;  // heu3: 1/deg of the sorted members (0 for degree 0)
+  u64* bkey;     // per block of 64 list positions: the largest member key (0 = none)
+  HL* L;
 };
 
 // Candidate keys, larger is chosen first, 0 = not a candidate.
@@ -100,135 +123,91 @@ struct HW {
 //   heu4: the complement of (degree in S, id), so the smallest pair is largest
 //   heu3: the bits of the (non-negative) double key, plus one; ties are broken
 //         by id when the chosen vertex is looked up
-__device__ __forceinline__ u64 kv2(const HW& w, u32 x) {
-  return w.sta[x] == 1 ? (((u64)(w.cnt[x] + 1) << 32) | x) : 0ull;
-}
-__device__ __forceinline__ u64 kv4(const HW& w, u32 x) {
-  return w.ins[x] ? ~(((u64)w.deg[x] << 32) | x) : 0ull;
-}
-__device__ __forceinline__ u64 kv3(const HW& w, u32 x) {
-  return w.sta[x] == 1 ? (u64)__double_as_longlong(w.key[x]) + 1ull : 0ull;
-}
-template <int MODE>
-__device__ __forceinline__ u64 kv(const HW& w, u32 x) {
-  return MODE == 2 ? kv2(w, x) : (MODE == 4 ? kv4(w, x) : kv3(w, x));
-}
-// block and group keys are raised by atomics at the L2; reads go past the L1
-__device__ __forceinline__ u64 hld64(u64* p) {
+__device__ __forceinline__ u64 k2(u32 cnt, u32 x) { return ((u64)(cnt + 1) << 32) | x; }
+__device__ __forceinline__ u64 k4(u32 deg, u32 x) { return ~(((u64)deg << 32) | x); }
+// block keys are raised by atomics at the L2; reads go past the L1
+__device__ __forceinline__ u64 hld64(const u64* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void hst64(u64* p, u64 v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// a member's key rose (or it joined): raise its block's and group's keys
 __device__ __forceinline__ void bump(HW& w, u32 p, u64 k) {
   atomicMax((unsigned long long*)&w.bkey[p >> 6], (unsigned long long)k);
-  atomicMax((unsigned long long*)&w.gkey[p >> 12], (unsigned long long)k);
+}
+__device__ __forceinline__ HV hget(const HW& w, u32 x) { return w.hv[x]; }
+
+// Places in the list for the wave's lanes with `on` (call on all lanes).
+__device__ __forceinline__ u32 push_pos(HW& w, bool on) {
+  const u64 b = __ballot(on);
+  u32 base = 0;
+  if (b) {
+    const int first = __ffsll((unsigned long long)b) - 1;
+    if (LANE == (u32)first) base = atomicAdd(&w.L->m, (u32)__popcll(b));
+    base = (u32)__shfl((int)base, first);
+  }
+  return base + (u32)__popcll(b & h_below());
 }
 
-// Exact keys of blocks b0 .. b0+cnt (eight per pass, so eight chains of
-// dependent loads are in flight), then of the groups they fall in.
-template <int MODE>
-__device__ void blocks_exact(HW& w, u32 b0, u32 cnt, u32 m) {
-  constexpr int U = 8;
-  for (u32 i0 = 0; i0 < cnt; i0 += U) {
-    u64 k[U];
-#pragma unroll
-    for (int t = 0; t < U; t++) {
-      const u32 p = (b0 + i0 + t) * 64 + LANE;
-      const bool in = i0 + t < cnt && p < m;
-      k[t] = in ? kv<MODE>(w, w.list[p]) : 0ull;
-    }
-#pragma unroll
-    for (int t = 0; t < U; t++) {
-      const u64 r = h_max64(k[t]);
-      if (LANE == 0 && i0 + t < cnt) hst64(&w.bkey[b0 + i0 + t], r);
-    }
+// Largest k and smallest mn over the block; one barrier.
+__device__ __forceinline__ void block_red(HL& L, u64& k, u32& mn) {
+  k = h_max64(k);
+  mn = h_min(mn);
+  if (LANE == 0) {
+    L.wmax[WAVE] = k;
+    L.wmin[WAVE] = mn;
   }
-  __threadfence();
-  hsync();
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < HEU_NW; i++) {
+    k = L.wmax[i] > k ? L.wmax[i] : k;
+    mn = min(mn, L.wmin[i]);
+  }
+}
+
+// This thread's share of the largest block key, without block bv.
+__device__ __forceinline__ u64 max_blocks(const HW& w, u32 m, u32 bv) {
   const u32 nblk = (m + 63) / 64;
-  for (u32 g = (b0 >> 6); g <= ((b0 + cnt - 1) >> 6); g++) {
-    const u32 b = g * 64 + LANE;
-    const u64 r = h_max64(b < nblk ? hld64(&w.bkey[b]) : 0ull);
-    if (LANE == 0) hst64(&w.gkey[g], r);
+  u64 k = 0;
+  for (u32 b0 = threadIdx.x; b0 < nblk; b0 += 4 * HEU_T) {
+    u64 x[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) x[t] = hld64(&w.bkey[min(b0 + t * HEU_T, nblk - 1)]);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+      if (b0 + t * HEU_T < nblk && b0 + t * HEU_T != bv && x[t] > k) k = x[t];
   }
-  __threadfence();
-  hsync();
-}
-
-// The largest key over all candidates (0 when there is none).
-__device__ __forceinline__ u64 top_key(HW& w, u32 m) {
-  const u32 ngrp = ((m + 63) / 64 + 63) / 64;
-  u64 best = 0;
-  for (u32 g = LANE; g < ngrp; g += 64) best = max(best, hld64(&w.gkey[g]));
-  return h_max64(best);
-}
-
-// heu3: the largest id among the candidates whose key is M.
-__device__ u32 find3(HW& w, u32 m, u64 M) {
-  const u32 nblk = (m + 63) / 64, ngrp = (nblk + 63) / 64;
-  u64 best = 0;
-  for (u32 g0 = 0; g0 < ngrp; g0 += 64) {
-    u64 gm = __ballot(g0 + LANE < ngrp && hld64(&w.gkey[g0 + LANE]) == M);
-    while (gm) {
-      const u32 g = g0 + (u32)(__ffsll((unsigned long long)gm) - 1);
-      gm &= gm - 1;
-      const u32 b1 = g * 64 + LANE;
-      u64 bm = __ballot(b1 < nblk && hld64(&w.bkey[b1]) == M);
-      while (bm) {
-        const u32 b = g * 64 + (u32)(__ffsll((unsigned long long)bm) - 1);
-        bm &= bm - 1;
-        const u32 p = b * 64 + LANE;
-        u64 c = 0;
-        if (p < m) {
-          const u32 x = w.list[p];
-          if (kv3(w, x) == M) c = (u64)x + 1;
-        }
-        best = max(best, h_max64(c));
-      }
-    }
-  }
-  return best ? (u32)(best - 1) : 0xffffffffu;
-}
-
-// Appends v to the candidate list (one lane per call site); its key is
-// raised by the caller.
-__device__ __forceinline__ u32 push_cand(HW& w, u32 v) {
-  const u32 p = atomicAdd(&w.L->m, 1u);
-  w.list[p] = v;
-  w.pos[v] = p;
-  return p;
-}
-
-// min over H = th[0..nH) of deg
-__device__ __forceinline__ u32 min_deg_h(HW& w, u32 nH) {
-  u32 mn = 0xffffffffu;
-  for (u32 i = LANE; i < nH; i += 64) mn = min(mn, w.deg[w.th[i]]);
-  return h_min(mn);
+  return k;
 }
 
 // Every array the run touched back to zero: the candidates' state and the
-// block and group keys.
-__device__ __forceinline__ void cleanup(HW& w) {
-  hsync();
-  const u32 m = hld(&w.L->m);
-  for (u32 i = LANE; i < m; i += 64) {
+// block keys.
+__device__ __forceinline__ void cleanup(HW& w, bool masks) {
+  __syncthreads();
+  const u32 m = w.L->m;
+  for (u32 i = threadIdx.x; i < m; i += HEU_T) {
     const u32 x = w.list[i];
-    w.sta[x] = 0;
-    w.ins[x] = 0;
-    w.cnt[x] = 0;
-    w.deg[x] = 0;
-    w.key[x] = 0.0;
+    w.hv[x] = HV{0, 0, 0, 0};
+    if (masks) {
+      w.key[x] = 0;
+      for (u32 k = 0; k < w.W; k++) w.mask[(u64)x * w.W + k] = 0;
+    }
   }
-  const u32 nblk = (m + 63) / 64, ngrp = (nblk + 63) / 64;
-  for (u32 b = LANE; b < nblk; b += 64) hst64(&w.bkey[b], 0ull);
-  for (u32 g = LANE; g < ngrp; g += 64) hst64(&w.gkey[g], 0ull);
-  __threadfence();
-  hsync();
-  if (LANE == 0) __hip_atomic_store(&w.L->m, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __threadfence();
-  hsync();
+  const u32 nblk = (m + 63) / 64;
+  for (u32 b = threadIdx.x; b < nblk; b += HEU_T) hst64(&w.bkey[b], 0ull);
+}
+
+// q as the only candidate, with key k.
+__device__ __forceinline__ void seed(HW& w, u32 q, u64 k) {
+  if (threadIdx.x == 0) {
+    HL& L = *w.L;
+    w.hv[q] = HV{0, 0, 0, 1};
+    w.list[0] = q;
+    hst64(&w.bkey[0], k);
+    L.m = 1;
+    L.dv[0] = L.dv[1] = L.rank[0] = L.rank[1] = L.best[0] = L.best[1] = 0;
+  }
+  __syncthreads();
 }
 
 // heu2 (inc/heuristic.h:8-120): H grows from q by the frontier vertex with
@@ -236,265 +215,305 @@ __device__ __forceinline__ void cleanup(HW& w) {
 // [N1, N2] by minimum degree (ties: the later one) is kept.
 __device__ __forceinline__ void heu2(HW& w, u32 N1, u32 N2, u32 q, u32* outH, u32 hcap,
                                      u32& osize, u32& okl) {
-  if (LANE == 0) {
-    w.sta[q] = 1;
-    bump(w, push_cand(w, q), kv2(w, q));
-  }
-  hsync();
+  HL& L = *w.L;
+  seed(w, q, k2(0, q));
   u32 nH = 0, tkl = 0, tsize = 0;
-  while (true) {
-    const u64 M = top_key(w, hld(&w.L->m));
-    if (M == 0) break;
-    const u32 v = (u32)M;
-    if (LANE == 0) {
+  u64 M = k2(0, q);
+  while (M) {
+    const u32 v = (u32)M, par = nH & 1;
+    const u32 b0 = w.off[v], e0 = w.off[v + 1], pv = w.hv[v].pos;
+    if (threadIdx.x == 0) {
       w.th[nH] = v;
-      w.sta[v] = 2;
+      w.hv[v].sta = 2;
+      L.dv[par ^ 1] = 0;
     }
     nH++;
-    hsync();
     u32 dv = 0;
-    const u32 b0 = w.off[v], e0 = w.off[v + 1];
-    for (u32 j = b0 + LANE; j < e0; j += 64) {
-      const u32 nb = w.adj[j];
-      const u32 c = w.cnt[nb] + 1;
-      w.cnt[nb] = c;
-      const u8 s = w.sta[nb];
-      const u64 k = ((u64)(c + 1) << 32) | nb;
-      if (s == 2) {
-        w.deg[nb] += 1;
-        dv++;
-      } else if (s == 0) {
-        w.sta[nb] = 1;
-        bump(w, push_cand(w, nb), k);
-      } else {
-        bump(w, w.pos[nb], k);
-      }
-    }
-    dv = h_sum(dv);
-    if (LANE == 0) w.deg[v] += dv;
-    hsync();
-    // v left the frontier: its block and group are recomputed exactly
-    blocks_exact<2>(w, w.pos[v] >> 6, 1, hld(&w.L->m));
-    if (nH >= N1) {
-      const u32 mn = min_deg_h(w, nH);
-      if (mn >= tkl) {
-        tkl = mn;
-        tsize = nH;
-      }
-    }
-    if (nH == N2) break;
-  }
-  for (u32 i = LANE; i < tsize && i < hcap; i += 64) outH[i] = w.th[i];
-  osize = tsize;
-  okl = tkl;
-  cleanup(w);
-}
-
-// Score of a frontier vertex nb whose degree is at most HEU_SMALL, by one
-// lane: 1/deg(w) over nb's H-neighbours w with deg(w) != 0 in ascending id
-// order, then deg(nb)/dmax.  nb has `target` H-neighbours (the count kept in
-// cnt during heu3), so the walk stops at the last of them.
-__device__ __forceinline__ double score_lane(const HW& w, u32 nb, u32 target) {
-  const u32 b = w.off[nb], e = w.off[nb + 1];
-  double sc = 0.0;
-  u32 found = 0;
-  for (u32 k = b; k < e && found < target; k++) {
-    const u32 x = w.adj[k];
-    if (w.sta[x] == 2) {
-      found++;
-      const u32 d = w.deg[x];
-      if (d != 0) sc += 1.0 / (double)d;
-    }
-  }
-  return sc + (double)(e - b) / (double)w.dmax;
-}
-
-// The same sum by the whole wave for a vertex of large degree: chunks of 64
-// entries, the chunk's terms added one after another in lane order, until
-// the last H-neighbour has been met.
-__device__ __forceinline__ double score_wave(const HW& w, u32 nb, u32 target) {
-  const u32 b = w.off[nb], e = w.off[nb + 1];
-  double sc = 0.0;
-  u32 found = 0;
-  for (u32 c = b; c < e && found < target; c += 64) {
-    const u32 k = c + LANE;
-    double t = 0.0;
-    bool inh = false, on = false;
-    if (k < e) {
-      const u32 x = w.adj[k];
-      if (w.sta[x] == 2) {
-        inh = true;
-        const u32 d = w.deg[x];
-        if (d != 0) {
-          t = 1.0 / (double)d;
-          on = true;
+    for (u32 j0 = b0; j0 < e0; j0 += 4 * HEU_T) {
+      u32 nb[4];
+      HV h[4];
+#pragma unroll
+      for (int t = 0; t < 4; t++) nb[t] = w.adj[min(j0 + t * HEU_T + threadIdx.x, e0 - 1)];
+#pragma unroll
+      for (int t = 0; t < 4; t++) h[t] = hget(w, nb[t]);
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        const bool in = j0 + t * HEU_T + threadIdx.x < e0;
+        const u32 c = h[t].cnt + 1;
+        const bool fresh = in && h[t].sta == 0;
+        const u32 p = push_pos(w, fresh);
+        if (in && h[t].sta == 2) {
+          w.hv[nb[t]].deg = h[t].deg + 1;
+          dv++;
+        } else if (fresh) {
+          w.hv[nb[t]] = HV{c, 0, p, 1};
+          w.list[p] = nb[t];
+          bump(w, p, k2(c, nb[t]));
+        } else if (in) {
+          w.hv[nb[t]].cnt = c;
+          bump(w, h[t].pos, k2(c, nb[t]));
         }
       }
     }
-    found += (u32)__popcll(__ballot(inh));
-    u64 msk = __ballot(on);
-    while (msk) {
-      const int i = __ffsll((unsigned long long)msk) - 1;
-      msk &= msk - 1;
-      sc += h_shfld(t, i);
+    dv = h_sum(dv);
+    if (LANE == 0 && dv) atomicAdd(&L.dv[par], dv);
+    __syncthreads();
+    // v's degree, v's block without v, the next choice, H's minimum degree
+    const u32 dvt = L.dv[par], m = L.m;
+    if (threadIdx.x == 0) w.hv[v].deg = dvt;
+    u64 k = max_blocks(w, m, pv >> 6);
+    if (WAVE == 0) {
+      const u32 p = (pv & ~63u) + LANE;
+      u64 kk = 0;
+      if (p < m) {
+        const u32 x = w.list[p];
+        const HV h = hget(w, x);
+        if (x != v && h.sta == 1) kk = k2(h.cnt, x);
+      }
+      kk = h_max64(kk);
+      if (LANE == 0) hst64(&w.bkey[pv >> 6], kk);
+      k = kk > k ? kk : k;
     }
+    u32 mn = 0xffffffffu;
+    if (nH >= N1)
+      for (u32 i = threadIdx.x; i < nH; i += HEU_T)
+        mn = min(mn, i == nH - 1 ? dvt : w.hv[w.th[i]].deg);
+    block_red(L, k, mn);
+    if (nH >= N1 && mn >= tkl) {
+      tkl = mn;
+      tsize = nH;
+    }
+    if (nH == N2) break;
+    M = k;
   }
-  return sc + (double)(e - b) / (double)w.dmax;
+  for (u32 i = threadIdx.x; i < tsize && i < hcap; i += HEU_T) outH[i] = w.th[i];
+  osize = tsize;
+  okl = tkl;
+  cleanup(w, false);
 }
 
-__device__ __forceinline__ void set_key3(HW& w, u32 nb, double sc) {
-  const u8 s = w.sta[nb];
-  if (s == 0) {
-    w.key[nb] = sc;
-    w.sta[nb] = 1;
-    bump(w, push_cand(w, nb), (u64)__double_as_longlong(sc) + 1ull);
-  } else if (sc > w.key[nb]) {
-    w.key[nb] = sc;
-    bump(w, w.pos[nb], (u64)__double_as_longlong(sc) + 1ull);
+// Sum of the terms of x's H-neighbours in ascending id order, for the wave's
+// 64 vertices at once: the sorted members go by one after another (64 of them
+// in the lanes' registers, read out with readlane), and a lane adds the term
+// when its vertex has the member's bit.  WN: words of a vertex's bits (0 = more
+// than four: a word is loaded when it is needed).
+template <int WN>
+__device__ __forceinline__ double walk_members(const HW& w, u32 nH, const u32* hj, u32 x, bool on) {
+  const u64* row = w.mask + (u64)x * w.W;
+  u64 mk[WN ? WN : 1];
+#pragma unroll
+  for (int i = 0; i < (WN ? WN : 1); i++) mk[i] = WN && on ? row[i] : 0ull;
+  double sc = 0.0;
+  for (u32 r0 = 0; r0 < nH; r0 += 64) {
+    const u32 cnt = min(64u, nH - r0), rl = r0 + min(LANE, cnt - 1);
+    const u64 tb = (u64)__double_as_longlong(w.term[rl]);
+    const u32 jl = hj[rl];
+    for (u32 r = 0; r < cnt; r++) {
+      const u32 j = __builtin_amdgcn_readlane(jl, r);
+      const u32 lo = __builtin_amdgcn_readlane((u32)tb, r);
+      const u32 hi = __builtin_amdgcn_readlane((u32)(tb >> 32), r);
+      u64 word = 0;
+      if (WN) {
+#pragma unroll
+        for (int i = 0; i < (WN ? WN : 1); i++)
+          if ((j >> 6) == (u32)i) word = mk[i];
+      } else if (on) {
+        word = row[j >> 6];
+      }
+      const double t = __longlong_as_double((long long)(((u64)hi << 32) | lo));
+      if ((word >> (j & 63)) & 1ull) sc += t;
+    }
   }
+  return sc;
 }
 
 // heu3 (inc/heuristic.h:125-239): H grows from q by the frontier vertex of
 // largest connection score (the largest score pushed for it).
 __device__ __forceinline__ void heu3(HW& w, u32 N1, u32 N2, u32 q, u32* outH, u32 hcap,
                                      u32& osize, u32& okl) {
-  if (LANE == 0) {
-    w.sta[q] = 1;
-    w.key[q] = 0.0;
-    bump(w, push_cand(w, q), kv3(w, q));
-  }
-  hsync();
-  u32 nH = 0, tkl = 0, tsize = 0;
+  HL& L = *w.L;
+  seed(w, q, 1ull);
+  if (threadIdx.x == 0) w.key[q] = 1ull;
+  u32 nH = 0, tkl = 0, tsize = 0, v = q;
   while (true) {
-    const u32 m = hld(&w.L->m);
-    const u64 M = top_key(w, m);
-    if (M == 0) break;
-    const u32 v = find3(w, m, M);
-    if (v == 0xffffffffu) break;  // keys and members disagree: stop (never seen)
-    if (LANE == 0) {
+    const u32 par = nH & 1, jn = nH;
+    const u32 b0 = w.off[v], e0 = w.off[v + 1], pv = w.hv[v].pos;
+    const u32 *hid = w.hsort + par * w.hrow, *hj = hid + 2 * w.hrow;
+    u32 *hidn = w.hsort + (par ^ 1) * w.hrow, *hjn = hidn + 2 * w.hrow;
+    if (threadIdx.x == 0) {
       w.th[nH] = v;
-      w.sta[v] = 2;
+      w.hv[v].sta = 2;
+      L.dv[par ^ 1] = 0;
+      L.rank[par ^ 1] = 0;
+      L.best[par] = 0;
     }
     nH++;
-    hsync();
-    const u32 b0 = w.off[v], e0 = w.off[v + 1];
+    // counts, degrees and bits of v's neighbours; H's sorted list with a gap
+    // for v
     u32 dv = 0;
-    for (u32 j = b0 + LANE; j < e0; j += 64) {
-      const u32 nb = w.adj[j];
-      w.cnt[nb] += 1;  // heu3 keeps each vertex's number of H-neighbours in cnt
-      if (w.sta[nb] == 2) {
-        w.deg[nb] += 1;
-        dv++;
+    for (u32 j0 = b0; j0 < e0; j0 += 4 * HEU_T) {
+      u32 nb[4];
+      HV h[4];
+      u64 mw[4];
+#pragma unroll
+      for (int t = 0; t < 4; t++) nb[t] = w.adj[min(j0 + t * HEU_T + threadIdx.x, e0 - 1)];
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        h[t] = hget(w, nb[t]);
+        mw[t] = w.mask[(u64)nb[t] * w.W + (jn >> 6)];
       }
-    }
-    dv = h_sum(dv);
-    if (LANE == 0) w.deg[v] += dv;
-    hsync();
-    // scores of v's neighbours outside H, against the degrees after v joined;
-    // a vertex whose only H-neighbour is v needs no walk: its sum is v's term
-    const u32 degv = w.deg[v];
-    const double termv = degv != 0 ? 1.0 / (double)degv : 0.0;
-    for (u32 c = b0; c < e0; c += 64) {
-      const u32 j = c + LANE;
-      u32 nb = 0, target = 0;
-      bool one = false, small = false, big = false;
-      if (j < e0) {
-        nb = w.adj[j];
-        if (w.sta[nb] != 2) {
-          target = w.cnt[nb];
-          const u32 dg = w.off[nb + 1] - w.off[nb];
-          one = target == 1;
-          small = !one && dg <= HEU_SMALL;
-          big = !one && !small;
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        if (j0 + t * HEU_T + threadIdx.x >= e0) continue;
+        if (h[t].sta == 2) {
+          w.hv[nb[t]].deg = h[t].deg + 1;
+          dv++;
+        } else {
+          w.hv[nb[t]].cnt = h[t].cnt + 1;
+          w.mask[(u64)nb[t] * w.W + (jn >> 6)] = mw[t] | (1ull << (jn & 63));
         }
       }
-      // a score reads only H's degrees, which no key update changes
-      if (one) {
-        const u32 dg = w.off[nb + 1] - w.off[nb];
-        set_key3(w, nb, (0.0 + termv) + (double)dg / (double)w.dmax);
+    }
+    u32 below = 0;
+    for (u32 i = threadIdx.x; i < jn; i += HEU_T) {
+      const u32 id = hid[i], to = i + (id > v ? 1u : 0u);
+      hidn[to] = id;
+      hjn[to] = hj[i];
+      below += id < v ? 1u : 0u;
+    }
+    dv = h_sum(dv);
+    below = h_sum(below);
+    if (LANE == 0) {
+      if (dv) atomicAdd(&L.dv[par], dv);
+      if (below) atomicAdd(&L.rank[par], below);
+    }
+    __syncthreads();
+    const u32 dvt = L.dv[par], rank = L.rank[par];
+    u32 mn = 0xffffffffu;
+    for (u32 i = threadIdx.x; i < nH; i += HEU_T) {
+      u32 d;
+      if (i == rank) {
+        hidn[i] = v;
+        hjn[i] = jn;
+        w.hv[v].deg = dvt;
+        d = dvt;
+      } else {
+        d = w.hv[hidn[i]].deg;
       }
-      if (small) set_key3(w, nb, score_lane(w, nb, target));
-      u64 bm = __ballot(big);
+      mn = min(mn, d);
+      w.term[i] = d ? 1.0 / (double)d : 0.0;
+    }
+    __syncthreads();
+    // scores of v's neighbours outside H, against the degrees after v joined;
+    // a vertex whose only H-neighbour is v needs no walk: its sum is v's term
+    const double termv = dvt != 0 ? 1.0 / (double)dvt : 0.0;
+    const u32 wn = (nH + 63) / 64;
+    for (u32 j0 = b0 + WAVE * 64; j0 < e0; j0 += HEU_T) {
+      const bool in = j0 + LANE < e0;
+      const u32 nb = w.adj[min(j0 + LANE, e0 - 1)];
+      const HV h = hget(w, nb);
+      const u32 dg = w.off[nb + 1] - w.off[nb];
+      const u64 old = w.key[nb];
+      const bool out = in && h.sta != 2, many = out && h.cnt > 1;
+      double sc = 0.0 + termv;
+      if (__ballot(many)) {
+        double s2;
+        if (wn == 1)
+          s2 = walk_members<1>(w, nH, hjn, nb, many);
+        else if (wn == 2)
+          s2 = walk_members<2>(w, nH, hjn, nb, many);
+        else if (wn <= 4 && w.W >= 4)
+          s2 = walk_members<4>(w, nH, hjn, nb, many);
+        else
+          s2 = walk_members<0>(w, nH, hjn, nb, many);
+        if (many) sc = s2;
+      }
+      sc += (double)dg / (double)w.dmax;
+      const u64 k = (u64)__double_as_longlong(sc) + 1ull;
+      const bool fresh = out && h.sta == 0;
+      const u32 p = push_pos(w, fresh);
+      if (fresh) {
+        w.hv[nb].pos = p;
+        w.hv[nb].sta = 1;
+        w.list[p] = nb;
+        w.key[nb] = k;
+        bump(w, p, k);
+      } else if (out && k > old) {
+        w.key[nb] = k;
+        bump(w, h.pos, k);
+      }
+    }
+    __syncthreads();
+    const u32 m = L.m;
+    u64 M = max_blocks(w, m, pv >> 6);
+    if (WAVE == 0) {
+      const u32 p = (pv & ~63u) + LANE;
+      u64 kk = 0;
+      if (p < m) {
+        const u32 x = w.list[p];
+        if (w.hv[x].sta == 1) kk = w.key[x];
+      }
+      kk = h_max64(kk);
+      if (LANE == 0) hst64(&w.bkey[pv >> 6], kk);
+      M = kk > M ? kk : M;
+    }
+    if (nH < N1) mn = 0xffffffffu;
+    block_red(L, M, mn);
+    if (nH >= N1 && mn >= tkl) {
+      tkl = mn;
+      tsize = nH;
+    }
+    if (nH == N2 || M == 0) break;
+    // the largest id among the candidates whose key is M
+    const u32 nblk = (m + 63) / 64;
+    for (u32 b0 = WAVE * 64; b0 < nblk; b0 += HEU_T) {
+      const u32 b = b0 + LANE;
+      u64 bm = __ballot(b < nblk && hld64(&w.bkey[min(b, nblk - 1)]) == M);
       while (bm) {
-        const int src = __ffsll((unsigned long long)bm) - 1;
+        const u32 p = (b0 + (u32)(__ffsll((unsigned long long)bm) - 1)) * 64 + LANE;
         bm &= bm - 1;
-        const u32 x = (u32)__shfl((int)nb, src);
-        const u32 tg = (u32)__shfl((int)target, src);
-        const double s2 = score_wave(w, x, tg);
-        if (LANE == 0) set_key3(w, x, s2);
+        if (p < m) {
+          const u32 x = w.list[p];
+          if (w.hv[x].sta == 1 && w.key[x] == M) atomicMax(&L.best[par], x + 1);
+        }
       }
     }
-    hsync();
-    blocks_exact<3>(w, w.pos[v] >> 6, 1, hld(&w.L->m));
-    if (nH >= N1) {
-      const u32 mn = min_deg_h(w, nH);
-      if (mn >= tkl) {
-        tkl = mn;
-        tsize = nH;
-      }
-    }
-    if (nH == N2) break;
+    __syncthreads();
+    const u32 best = L.best[par];
+    if (best == 0) break;  // keys and members disagree: stop (never seen)
+    v = best - 1;
   }
-  for (u32 i = LANE; i < tsize && i < hcap; i += 64) outH[i] = w.th[i];
+  for (u32 i = threadIdx.x; i < tsize && i < hcap; i += HEU_T) outH[i] = w.th[i];
   osize = tsize;
   okl = tkl;
-  cleanup(w);
+  cleanup(w, true);
 }
 
 // heu4 (inc/heuristic.h:242-317): S = q and its neighbours; peel the vertex
 // of smallest (degree in S, id) until N1 remain, keeping the peel prefix
-// whose popped degree is the largest with |S left| in [N1, N2].
-__device__ __forceinline__ void heu4(HW& w, u32 N1, u32 N2, u32 q, u32* outH, u32 hcap, u32& osize, u32& okl) {
-  osize = 0;
-  okl = 0;
-  const u32 qb = w.off[q], qe = w.off[q + 1];
-  if (qe - qb < N1 - 1u) return;
-  const u32 m = 1 + (qe - qb);
-  if (LANE == 0) {
-    w.list[0] = q;
-    w.pos[q] = 0;
-    w.ins[q] = 1;
-    __hip_atomic_store(&w.L->m, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  for (u32 j = qb + LANE; j < qe; j += 64) {
-    const u32 x = w.adj[j];
-    w.list[1 + (j - qb)] = x;
-    w.pos[x] = 1 + (j - qb);
-    w.ins[x] = 1;
-  }
-  hsync();
-  // degree of each member inside S (q: one more, as the reference counts it)
-  for (u32 i0 = 0; i0 < m; i0 += 64) {
-    const u32 i = i0 + LANE;
-    u32 x = 0, b = 0, e = 0;
-    if (i < m) {
-      x = w.list[i];
-      b = w.off[x];
-      e = w.off[x + 1];
-    }
-    const bool big = i < m && (e - b) > HEU_SMALL;
-    if (i < m && !big) {
-      u32 c = 0;
-      for (u32 k = b; k < e; k++) c += w.ins[w.adj[k]];
-      w.deg[x] = c + (x == q ? 1u : 0u);
-    }
-    u64 bm = __ballot(big);
-    while (bm) {
-      const int src = __ffsll((unsigned long long)bm) - 1;
-      bm &= bm - 1;
-      const u32 bx = (u32)__shfl((int)x, src), bb = (u32)__shfl((int)b, src),
-                be = (u32)__shfl((int)e, src);
-      u32 c = 0;
-      for (u32 k = bb + LANE; k < be; k += 64) c += w.ins[w.adj[k]];
-      c = h_sum(c);
-      if (LANE == 0) w.deg[bx] = c + (bx == q ? 1u : 0u);
-    }
-  }
-  hsync();
-  blocks_exact<4>(w, 0, (m + 63) / 64, m);
+// whose popped degree is the largest with |S left| in [N1, N2].  The degrees
+// are counted by the whole block; the peeling, one vertex after another, is
+// one wave's, without block barriers.  Up to 4,096 members' block keys are in
+// LDS.
+template <bool INLDS>
+__device__ __forceinline__ void peel4(HW& w, u32 m, u32 N1, u32 N2, u32 q) {
+  HL& L = *w.L;
+  const u32 nblk = (m + 63) / 64;
   u32 nr = 0, rmv_idx = 0, mindeg = 0;
   while (true) {
-    const u64 M = top_key(w, m);
+    u64 M = 0;
+    if (INLDS) {
+      M = LANE < nblk ? L.bk[LANE] : 0ull;
+    } else {
+      for (u32 b0 = LANE; b0 < nblk; b0 += 256) {
+        u64 x[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) x[t] = hld64(&w.bkey[min(b0 + 64u * t, nblk - 1)]);
+#pragma unroll
+        for (int t = 0; t < 4; t++) M = x[t] > M ? x[t] : M;
+      }
+    }
+    M = h_max64(M);
     if (M == 0) break;
     const u64 best = ~M;
     const u32 v = (u32)best;
@@ -506,73 +525,174 @@ __device__ __forceinline__ void heu4(HW& w, u32 N1, u32 N2, u32 q, u32* outH, u3
       rmv_idx = nr;
     }
     if (remain == N1) break;
+    // v's block without v, from the degrees before v's neighbours lose it
+    // (their keys only rise), while v's adjacency is on its way
+    const u32 b0 = w.off[v], e0 = w.off[v + 1], bv = w.hv[v].pos >> 6;
+    const u32 p = bv * 64 + LANE;
+    u32 x = w.adj[min(b0 + LANE, e0 - 1)];
+    const u32 y = w.list[min(p, m - 1)];
+    const HV hy = hget(w, y);
+    u64 kk = h_max64(p < m && y != v && hy.sta ? k4(hy.deg, y) : 0ull);
     if (LANE == 0) {
-      w.ins[v] = 0;
+      w.hv[v].sta = 0;
       w.rmv[nr] = v;
+      if (INLDS)
+        L.bk[bv] = kk;
+      else
+        hst64(&w.bkey[bv], kk);
     }
     nr++;
-    hsync();
-    const u32 b0 = w.off[v], e0 = w.off[v + 1];
-    for (u32 j = b0 + LANE; j < e0; j += 64) {
-      const u32 x = w.adj[j];
-      if (w.ins[x]) {
-        const u32 d2 = w.deg[x] - 1;
-        w.deg[x] = d2;
-        bump(w, w.pos[x], ~(((u64)d2 << 32) | x));
+    // the key is in place before the rises below reach it
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    for (u32 j0 = b0; j0 < e0; j0 += 64) {
+      const bool in = j0 + LANE < e0;
+      const u32 xn = w.adj[min(j0 + 64 + LANE, e0 - 1)];
+      const HV h = hget(w, x);
+      if (in && h.sta) {
+        w.hv[x].deg = h.deg - 1;
+        const u64 k = k4(h.deg - 1, x);
+        if (INLDS)
+          atomicMax((unsigned long long*)&L.bk[h.pos >> 6], (unsigned long long)k);
+        else
+          bump(w, h.pos, k);
       }
+      x = xn;
     }
-    hsync();
-    blocks_exact<4>(w, w.pos[v] >> 6, 1, m);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
   }
-  // H = S without the first rmv_idx peeled vertices, in S order
-  for (u32 i = LANE; i < m; i += 64) w.ins[w.list[i]] = 1;
-  hsync();
-  for (u32 i = LANE; i < rmv_idx; i += 64) w.ins[w.rmv[i]] = 0;
-  hsync();
-  u32 base = 0;
-  for (u32 i0 = 0; i0 < m; i0 += 64) {
-    const u32 i = i0 + LANE;
-    const bool keep = i < m && w.ins[w.list[i]];
-    const u64 bal = __ballot(keep);
-    if (keep) {
-      const u32 p = base + (u32)__popcll(bal & ((1ull << LANE) - 1ull));
-      if (p < hcap) outH[p] = w.list[i];
-    }
-    base += (u32)__popcll(bal);
+  if (LANE == 0) {
+    L.mindeg = mindeg;
+    L.remove = rmv_idx;
   }
-  osize = base;
-  okl = mindeg;
-  cleanup(w);
 }
 
-// Three waves per query, one per construction (block 3i + c runs heu2,
-// heu3 or heu4 of query i in its own workspace).  No LDS: the wave's
-// counter lives in its workspace, so the kernel also finds room on CUs
-// whose LDS the search kernel holds.
-__global__ void __launch_bounds__(64) __attribute__((flatten)) scs_heu_kernel(HeuArgs A) {
+__device__ __forceinline__ void heu4(HW& w, u32 N1, u32 N2, u32 q, u32* outH, u32 hcap, u32& osize,
+                                     u32& okl) {
+  HL& L = *w.L;
+  osize = 0;
+  okl = 0;
+  const u32 qb = w.off[q], qe = w.off[q + 1];
+  if (qe - qb < N1 - 1u) return;
+  const u32 m = 1 + (qe - qb), nblk = (m + 63) / 64;
+  const bool inlds = nblk <= HEU_LDSB;
+  for (u32 i = threadIdx.x; i < m; i += HEU_T) {
+    const u32 x = i ? w.adj[qb + i - 1] : q;
+    w.list[i] = x;
+    w.hv[x] = HV{0, 0, i, 1};
+  }
+  if (threadIdx.x == 0) L.m = m;
+  __syncthreads();
+  // degree of each member inside S (q: one more, as the reference counts it)
+  for (u32 i0 = WAVE * 64; i0 < m; i0 += HEU_T) {
+    const u32 i = i0 + LANE;
+    const bool on = i < m;
+    u32 x = 0, b = 0, e = 0, c = 0;
+    if (on) {
+      x = w.list[i];
+      b = w.off[x];
+      e = w.off[x + 1];
+    }
+    const bool big = on && (e - b) > HEU_SMALL;
+    if (on && !big) {
+      for (u32 k = b; k < e; k += 4) {
+        u32 y[4], s[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) y[t] = w.adj[min(k + t, e - 1)];
+#pragma unroll
+        for (int t = 0; t < 4; t++) s[t] = w.hv[y[t]].sta;
+#pragma unroll
+        for (int t = 0; t < 4; t++) c += k + t < e ? s[t] : 0u;
+      }
+    }
+    u64 bm = __ballot(big);
+    while (bm) {
+      const int src = __ffsll((unsigned long long)bm) - 1;
+      bm &= bm - 1;
+      const u32 bb = (u32)__shfl((int)b, src), be = (u32)__shfl((int)e, src);
+      u32 cc = 0;
+      for (u32 k = bb; k < be; k += 256) {
+        u32 y[4], s[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) y[t] = w.adj[min(k + 64u * t + LANE, be - 1)];
+#pragma unroll
+        for (int t = 0; t < 4; t++) s[t] = w.hv[y[t]].sta;
+#pragma unroll
+        for (int t = 0; t < 4; t++) cc += k + 64u * t + LANE < be ? s[t] : 0u;
+      }
+      cc = h_sum(cc);
+      if (LANE == (u32)src) c = cc;
+    }
+    c += x == q ? 1u : 0u;
+    if (on) w.hv[x].deg = c;
+    const u64 kk = h_max64(on ? k4(c, x) : 0ull);
+    if (LANE == 0) {
+      if (inlds)
+        L.bk[i0 >> 6] = kk;
+      else
+        hst64(&w.bkey[i0 >> 6], kk);
+    }
+  }
+  __syncthreads();
+  if (WAVE == 0) {
+    if (inlds)
+      peel4<true>(w, m, N1, N2, q);
+    else
+      peel4<false>(w, m, N1, N2, q);
+  }
+  __syncthreads();
+  const u32 rmv_idx = L.remove, mindeg = L.mindeg;
+  // H = S without the first rmv_idx peeled vertices, in S order
+  for (u32 i = threadIdx.x; i < m; i += HEU_T) w.hv[w.list[i]].sta = 1;
+  __syncthreads();
+  for (u32 i = threadIdx.x; i < rmv_idx; i += HEU_T) w.hv[w.rmv[i]].sta = 0;
+  __syncthreads();
+  if (WAVE == 0) {
+    u32 base = 0;
+    for (u32 i0 = 0; i0 < m; i0 += 256) {
+      u32 x[4], s[4];
+#pragma unroll
+      for (int t = 0; t < 4; t++) x[t] = w.list[min(i0 + 64u * t + LANE, m - 1)];
+#pragma unroll
+      for (int t = 0; t < 4; t++) s[t] = w.hv[x[t]].sta;
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        const bool keep = i0 + 64u * t + LANE < m && s[t];
+        const u64 bal = __ballot(keep);
+        const u32 p = base + (u32)__popcll(bal & h_below());
+        if (keep && p < hcap) outH[p] = x[t];
+        base += (u32)__popcll(bal);
+      }
+    }
+  }
+  osize = m - rmv_idx;
+  okl = mindeg;
+  cleanup(w, false);
+}
+
+// Three blocks per query, one per construction (block 3i + c runs heu2, heu3
+// or heu4 of query i in its own workspace).
+__global__ void __launch_bounds__(HEU_T, 4) scs_heu_kernel(HeuArgs A) {
+  __shared__ HL L;
   const u32 bi = blockIdx.x, qi = bi / 3, which = bi % 3;
   if (qi >= A.nq) return;
-  u8* base = A.ws + (u64)bi * A.lay.stride;
+  u8* const z = A.zs + (u64)qi * A.lay.zstride + A.lay.zpart[which];
+  u8* const g = A.gs + (u64)qi * A.lay.gstride + A.lay.gpart[which];
   HW w;
   w.off = A.off;
   w.adj = A.adj;
   w.n = A.n;
   w.dmax = A.dmax;
-  w.sta = base + A.lay.sta;
-  w.ins = base + A.lay.ins;
-  w.cnt = (u32*)(base + A.lay.cnt);
-  w.deg = (u32*)(base + A.lay.deg);
-  w.key = (double*)(base + A.lay.key);
-  w.pos = (u32*)(base + A.lay.pos);
-  w.list = (u32*)(base + A.lay.list);
-  w.rmv = (u32*)(base + A.lay.rmv);
-  w.th = (u32*)(base + A.lay.th);
-  w.bkey = (u64*)(base + A.lay.bkey);
-  w.gkey = (u64*)(base + A.lay.gkey);
-  w.L = (HeuLds*)(base + A.lay.lds);
-  if (LANE == 0) __hip_atomic_store(&w.L->m, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __threadfence();
-  hsync();
+  w.W = A.lay.words;
+  w.hv = (HV*)z;
+  w.bkey = (u64*)(z + A.lay.bkey);
+  w.key = (u64*)(z + A.lay.key);
+  w.mask = (u64*)(z + A.lay.mask);
+  w.list = (u32*)g;
+  w.th = w.rmv = (u32*)(g + A.lay.th);  // heu2 and heu3 use one, heu4 the other
+  w.hsort = (u32*)(g + A.lay.hsort);
+  w.hrow = A.lay.hrow;
+  w.term = (double*)(g + A.lay.term);
+  w.L = &L;
   const u32 l = A.ql[qi], h = A.qh[qi], q = A.qq[qi];
   u32* out = A.H3 + (u64)bi * A.hcap;
   u32 sz = 0, kk = 0;
@@ -582,7 +702,7 @@ __global__ void __launch_bounds__(64) __attribute__((flatten)) scs_heu_kernel(He
     heu3(w, l, h, q, out, A.hcap, sz, kk);
   else
     heu4(w, l, h, q, out, A.hcap, sz, kk);
-  if (LANE == 0) {
+  if (threadIdx.x == 0) {
     A.kl3[bi] = kk;
     A.hs3[bi] = sz;
   }
@@ -607,31 +727,39 @@ __global__ void __launch_bounds__(64) scs_heu_pick(HeuArgs A) {
 
 static u64 heu_al(u64 x) { return (x + 255) & ~255ull; }
 
-extern "C" HeuLayout scs_heu_layout(u32 n, u32 hcap) {
+// Workspace of one query whose h is at most hmax, in three parts (heu2, heu3,
+// heu4) of two areas: the arrays a block finds zeroed and leaves zeroed, whose
+// layout depends on hmax, and the others, whose layout does not, so that runs
+// with different hmax can share a workspace.
+extern "C" HeuLayout scs_heu_layout(u32 n, u32 hmax) {
   HeuLayout L{};
-  const u64 nblk = (n + 63) / 64 + 1;
-  u64 o = 0;
-  L.sta = o; o = heu_al(o + n);
-  L.ins = o; o = heu_al(o + n);
-  L.cnt = o; o = heu_al(o + 4ull * n);
-  L.deg = o; o = heu_al(o + 4ull * n);
+  L.words = (hmax + 63) / 64;
+  if (L.words == 3) L.words = 4;  // the walk takes 1, 2 or 4 words in registers
+  u64 o = heu_al(16ull * n);  // records first
+  L.bkey = o; o = heu_al(o + 8ull * ((n + 63) / 64 + 1));
+  const u64 z24 = o;
   L.key = o; o = heu_al(o + 8ull * n);
-  L.pos = o; o = heu_al(o + 4ull * n);
-  L.list = o; o = heu_al(o + 4ull * (n + 64));
-  L.rmv = o; o = heu_al(o + 4ull * (n + 64));
-  L.th = o; o = heu_al(o + 4ull * (4ull * hcap + 64));
-  L.bkey = o; o = heu_al(o + 8 * nblk);
-  L.gkey = o; o = heu_al(o + 8 * (nblk / 64 + 2));
-  L.lds = o; o = heu_al(o + sizeof(HeuLds));
-  L.stride = o;
+  L.mask = o; o = heu_al(o + 8ull * L.words * n);
+  L.zpart[1] = z24;
+  L.zpart[2] = z24 + o;
+  L.zstride = 2 * z24 + o;
+  L.hrow = SCS_MAX_H + 24;
+  o = heu_al(4ull * (n + 64));  // the list first
+  L.th = o; o = heu_al(o + 4ull * (SCS_MAX_H + 64));
+  const u64 g2 = o, g4 = heu_al(L.th + 4ull * (n + 64));
+  L.hsort = o; o = heu_al(o + 16ull * L.hrow);
+  L.term = o; o = heu_al(o + 8ull * L.hrow);
+  L.gpart[1] = g2;
+  L.gpart[2] = g2 + o;
+  L.gstride = g2 + o + g4;
   return L;
 }
 
-// ws holds 3 * nq workspaces; kl3/hs3/H3 hold the three constructions'
+// zs and gs hold nq workspaces; kl3/hs3/H3 hold the three constructions'
 // results of each query, kl/hsize/H the picked one.
 extern "C" hipError_t scs_launch_heu(const u32* off, const u32* adj, u32 n, u32 dmax, u32 nq,
-                                     const u32* ql, const u32* qh, const u32* qq, u8* ws,
-                                     HeuLayout lay, u32 hcap, u32* kl, u32* hsize, u32* H,
+                                     const u32* ql, const u32* qh, const u32* qq, u8* zs,
+                                     u8* gs, HeuLayout lay, u32 hcap, u32* kl, u32* hsize, u32* H,
                                      u32* kl3, u32* hs3, u32* H3, hipStream_t s) {
   HeuArgs A;
   A.off = off;
@@ -643,7 +771,8 @@ extern "C" hipError_t scs_launch_heu(const u32* off, const u32* adj, u32 n, u32 
   A.ql = ql;
   A.qh = qh;
   A.qq = qq;
-  A.ws = ws;
+  A.zs = zs;
+  A.gs = gs;
   A.lay = lay;
   A.kl = kl;
   A.hsize = hsize;
@@ -651,7 +780,7 @@ extern "C" hipError_t scs_launch_heu(const u32* off, const u32* adj, u32 n, u32 
   A.kl3 = kl3;
   A.hs3 = hs3;
   A.H3 = H3;
-  scs_heu_kernel<<<3 * nq, 64, 0, s>>>(A);
+  scs_heu_kernel<<<3 * nq, HEU_T, 0, s>>>(A);
   scs_heu_pick<<<nq, 64, 0, s>>>(A);
   return hipGetLastError();
 }

@@ -221,12 +221,11 @@ struct EngineArgs {
   u32 no_bitmaps;      // 1 = no LDS bitmaps (status from device memory only)
 };
 
-// GPU greedy heuristic (scs_heu.hip): byte offsets of one wave's workspace
-// (every n-sized array is all-zero between queries) and its two counters.
+// GPU greedy heuristic (scs_heu.hip): byte offsets inside one construction's
+// part of a query's two work areas (z: zero between queries, g: not), of the
+// parts inside the areas, the areas' sizes per query, and words of heu3's bits.
 struct HeuLayout {
-  u64 sta, ins, cnt, deg, key, pos, list, rmv, th, bkey, gkey, lds, stride;
-};
-struct HeuLds {
-  u32 m;  // candidates in the list
-  u32 pad[3];
+  u64 bkey, key, mask, zpart[3], zstride;
+  u64 th, hsort, term, gpart[3], gstride;
+  u32 words, hrow;
 };
