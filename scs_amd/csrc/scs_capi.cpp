@@ -28,24 +28,24 @@ int scs_core_run(const i64* off, const int32_t* adj, u32 n, u32* core, u32* tmp,
                  hipStream_t s);
 u64 scs_core_words(u32 n);
 hipError_t scs_launch_ms_init(u32 n, const u32* core, const MsBatch* B, u64* elig, u64* vis,
-                              u64* fr, u64* nf, u32* flags, u32 nflags, unsigned long long* bytes,
-                              hipStream_t s);
+                              u64* fr, u64* nf, u64* xf, u32* flags, u32 nflags,
+                              unsigned long long* bytes, hipStream_t s);
 hipError_t scs_launch_ms_push0(const i64* off, const int32_t* adj, u32 nb, const MsBatch* B,
                                u64 act, const u64* elig, u64* vis, u64* nf, u16* dist16,
                                u32* flag0, unsigned long long* bytes, hipStream_t s);
 hipError_t scs_launch_ms_seed(const MsBatch* B, u64* vis, u64* fr, u16* dist16, hipStream_t s);
-hipError_t scs_launch_ms_level(const i64* off, const int32_t* adj, u32 n, u32 level, u64 act,
-                               const u64* elig, u64* vis, const u64* fr, u64* nf, u16* dist16,
+hipError_t scs_launch_ms_level(const int32_t* adj, const MsUnit* units, u32 nunits,
+                               const MsHub* hubs, u32 nhubs, u32 level, u64 act, const u64* elig,
+                               u64* vis, const u64* fr, u64* nf, u64* clr, u16* dist16,
                                const u32* flag_prev, u32* flag_cur, unsigned long long* bytes,
                                hipStream_t s);
-hipError_t scs_launch_ms_count(u32 n, u32 G, const u64* vis, u64 valid, u32* gcnt,
-                               unsigned long long* bytes, hipStream_t s);
-hipError_t scs_launch_ms_bscan(u32 nb, u32 G, u32* gcnt, u32* tot, unsigned long long* bytes,
-                               hipStream_t s);
+hipError_t scs_launch_ms_count(u32 n, u32 G, u64* vis, const u64* lf, u64 valid, u32* gcnt,
+                               u32* cbase, u32* tot, unsigned long long* bytes, hipStream_t s);
+u64 scs_ms_count_rows(u32 G);
 hipError_t scs_launch_ms_gdist(u32 n, u32 G, const u64* vis, u64 gmask, const u16* dist16,
                                const MsBatch* B, unsigned long long* bytes, hipStream_t s);
 hipError_t scs_launch_ms_scatter(u32 n, u32 G, const u64* vis, u64 valid, const u32* gcnt,
-                                 const u32* core, const u16* dist16, const MsBatch* B, u32* locid,
+                                 const u32* cbase, const u32* core, const u16* dist16, const MsBatch* B, u32* locid,
                                  u32* qloc, unsigned long long* bytes, hipStream_t s);
 hipError_t scs_launch_ms_degree(const int32_t* adj, const MsUnit* units, u32 nunits,
                                 const MsHub* hubs, u32 nhubs, const u64* vis, u64 valid,
@@ -54,8 +54,8 @@ hipError_t scs_launch_ms_degree(const int32_t* adj, const MsUnit* units, u32 nun
 hipError_t scs_launch_ms_scan_loff(u32 nb, const MsBatch* B, u32* tot, u64 valid, u32 cmax,
                                    u32* csum, unsigned long long* bytes, hipStream_t s);
 hipError_t scs_launch_ms_fill(const int32_t* adj, const MsUnit* units, u32 nunits,
-                              const u64* vis, u64 valid, const u32* locid, const MsBatch* B,
-                              const u32* hubcnt, unsigned long long* bytes, hipStream_t s);
+                              const u64* vis, u64 valid, u64 packed, const u32* locid,
+                              const MsBatch* B, const u32* hubcnt, unsigned long long* bytes, hipStream_t s);
 hipError_t scs_launch_epoch(const EngineArgs* A, hipStream_t s);
 hipError_t scs_launch_slot_write(const QuerySlot* stage, const u32* idx, const u32* wit, u32 n,
                                  QuerySlot* slots, u32* witness, hipStream_t s);
@@ -407,6 +407,7 @@ struct HostSlot {
   PendingQuery pq;
   std::vector<u32> seed_witness;  // heuristic H, copied into the slot at admission
   u32 kl0 = 0, ku = 0, K = 0;
+  u32 nnz = 0;  // local adjacency entries (0 for a whole-graph query)
   u64 a_off = 0, a_len = 0, b_off = 0, b_len = 0;
   u64 need = 0;  // arena bytes known to be needed when admission was refused
   bool whole = false;     // searches the resident graph's CSR (no local graph)
@@ -430,10 +431,11 @@ struct scs_engine {
   EngineGlobals* d_glob = nullptr;
   EngineArgs args{};
   // batched preprocessing (bit b of a mask = query b of the batch)
-  u64 *d_elig = nullptr, *d_vis = nullptr, *d_fr = nullptr, *d_nf = nullptr;
+  u64 *d_elig = nullptr, *d_vis = nullptr, *d_fr = nullptr, *d_nf = nullptr, *d_xf = nullptr;
   u16* d_dist16 = nullptr;   // [n][64] BFS distance per query
-  u32* d_locid64 = nullptr;  // [n][64] local id per query
-  u32* d_gcnt = nullptr;     // [ceil(n/64)][64] group counts, then bases
+  u32* d_locid64 = nullptr;  // [n][up to 64] local id per query
+  u32* d_gcnt = nullptr;     // [ceil(n/64)][64] counts before each group in its chunk
+  u32* d_cbase = nullptr;    // [chunks][64] chunk counts, then bases
   MsUnit* d_units = nullptr;  // adjacency units of every vertex
   MsHub* d_hubs = nullptr;    // vertices with more than one unit
   u32 nunits = 0, nhubs = 0;
@@ -600,11 +602,13 @@ extern "C" int scs_engine_create(scs_graph* g, const scs_params* pin, scs_engine
   if (hipMalloc(&E->d_glob, sizeof(EngineGlobals)) != hipSuccess) return fail(SCS_ENOMEM);
   const u32 n1 = std::max<u32>(n, 1);
   const u64 G = (n1 + 63) / 64;
-  for (u64** b : {&E->d_elig, &E->d_vis, &E->d_fr, &E->d_nf})
+  for (u64** b : {&E->d_elig, &E->d_vis, &E->d_fr, &E->d_nf, &E->d_xf})
     if (hipMalloc(b, sizeof(u64) * n1) != hipSuccess) return fail(SCS_ENOMEM);
   if (hipMalloc(&E->d_dist16, sizeof(u16) * 64 * (u64)n1) != hipSuccess) return fail(SCS_ENOMEM);
   if (hipMalloc(&E->d_locid64, sizeof(u32) * 64 * (u64)n1) != hipSuccess) return fail(SCS_ENOMEM);
   if (hipMalloc(&E->d_gcnt, sizeof(u32) * 64 * G) != hipSuccess) return fail(SCS_ENOMEM);
+  if (hipMalloc(&E->d_cbase, sizeof(u32) * 64 * scs_ms_count_rows((u32)G)) != hipSuccess)
+    return fail(SCS_ENOMEM);
   {
     // adjacency units: one per vertex, or ceil(deg / MS_UNIT) for a hub
     std::vector<MsUnit> units;
@@ -771,8 +775,8 @@ extern "C" void scs_engine_destroy(scs_engine* E) {
   if (E->ps) (void)hipStreamSynchronize(E->ps);
   E->heu_gpu.release();
   void* ptrs[] = {E->d_slots, E->d_witness, E->d_wave, E->d_pool_seq, E->d_pool_data,
-                  E->d_pool_pos, E->d_glob, E->d_elig, E->d_vis, E->d_fr, E->d_nf, E->d_dist16,
-                  E->d_locid64, E->d_gcnt, E->d_units, E->d_hubs, E->d_hubcnt, E->d_csum,
+                  E->d_pool_pos, E->d_glob, E->d_elig, E->d_vis, E->d_fr, E->d_nf, E->d_xf,
+                  E->d_dist16, E->d_locid64, E->d_gcnt, E->d_cbase, E->d_units, E->d_hubs, E->d_hubcnt, E->d_csum,
                   E->d_flags, E->d_tot, E->d_batch, E->d_admit,
                   E->d_prepbytes, E->d_arena, E->d_model, E->d_trace, E->d_trace_cnt};
   for (void* q : ptrs)
@@ -923,20 +927,20 @@ static int prep_batch(scs_engine* E, const u32* sis, const u32* kl0s, const u32*
   HIPCHK(hipEventRecord(E->pe0, s));
   HIPCHK(hipMemcpyAsync(E->d_batch, &B, sizeof(MsBatch), hipMemcpyHostToDevice, s));
   HIPCHK(scs_launch_ms_init(n, E->g->d_core, E->d_batch, E->d_elig, E->d_vis, E->d_fr, E->d_nf,
-                            E->d_flags, SCS_MS_LEVELS, E->d_prepbytes, s));
+                            E->d_xf, E->d_flags, SCS_MS_LEVELS, E->d_prepbytes, s));
   HIPCHK(scs_launch_ms_seed(E->d_batch, E->d_vis, E->d_fr, E->d_dist16, s));
   // BFS levels; a level that finds nothing ends the later ones on the
   // device, and the host checks every 8 levels
-  u64 *fr = E->d_fr, *nf = E->d_nf;
+  // level L reads buf[L % 3], writes the next and clears the hubs of the third
+  u64* const buf[3] = {E->d_fr, E->d_nf, E->d_xf};
   u32 L = 0;
   if (maxU > 0) {
     // level 0 pushes from the query vertices (top-down)
     u64 act = 0;
     for (u32 b = 0; b < cnt; b++)
       if (ubd[b] > 0) act |= 1ull << b;
-    HIPCHK(scs_launch_ms_push0(off, adj, cnt, E->d_batch, act, E->d_elig, E->d_vis, nf,
+    HIPCHK(scs_launch_ms_push0(off, adj, cnt, E->d_batch, act, E->d_elig, E->d_vis, buf[1],
                                E->d_dist16, E->d_flags, E->d_prepbytes, s));
-    std::swap(fr, nf);
     L = 1;
   }
   while (L < maxU) {
@@ -945,9 +949,10 @@ static int prep_batch(scs_engine* E, const u32* sis, const u32* kl0s, const u32*
       u64 act = 0;
       for (u32 b = 0; b < cnt; b++)
         if (ubd[b] > L) act |= 1ull << b;
-      HIPCHK(scs_launch_ms_level(off, adj, n, L, act, E->d_elig, E->d_vis, fr, nf, E->d_dist16,
-                                 E->d_flags + (L ? L - 1 : 0), E->d_flags + L, E->d_prepbytes, s));
-      std::swap(fr, nf);
+      HIPCHK(scs_launch_ms_level(adj, E->d_units, E->nunits, E->d_hubs, E->nhubs, L, act,
+                                 E->d_elig, E->d_vis, buf[L % 3], buf[(L + 1) % 3],
+                                 buf[(L + 2) % 3], E->d_dist16, E->d_flags + (L ? L - 1 : 0),
+                                 E->d_flags + L, E->d_prepbytes, s));
     }
     if (L >= maxU) break;
     HIPCHK(hipMemcpyAsync(E->h_tot, E->d_flags + (L - 1), sizeof(u32), hipMemcpyDeviceToHost, s));
@@ -955,8 +960,8 @@ static int prep_batch(scs_engine* E, const u32* sis, const u32* kl0s, const u32*
     if (E->h_tot[0] == 0) break;
   }
   // kept sets: group counts, per-query bases and sizes
-  HIPCHK(scs_launch_ms_count(n, G, E->d_vis, all, E->d_gcnt, E->d_prepbytes, s));
-  HIPCHK(scs_launch_ms_bscan(cnt, G, E->d_gcnt, E->d_tot, E->d_prepbytes, s));
+  HIPCHK(scs_launch_ms_count(n, G, E->d_vis, buf[L % 3], all, E->d_gcnt, E->d_cbase, E->d_tot,
+                             E->d_prepbytes, s));
   HIPCHK(hipMemcpyAsync(E->h_tot, E->d_tot, sizeof(u32) * 64, hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
   u64 valid = 0, gmask = 0;
@@ -969,6 +974,7 @@ static int prep_batch(scs_engine* E, const u32* sis, const u32* kl0s, const u32*
     HostSlot& hs = E->slots[sis[i]];
     const u32 K = E->h_tot[b];
     hs.K = K;
+    hs.nnz = 0;
     hs.whole = false;
     if (K > E->kcap || K == 0) {
       rcs[i] = SCS_EBIG;
@@ -1009,8 +1015,9 @@ static int prep_batch(scs_engine* E, const u32* sis, const u32* kl0s, const u32*
   if (valid | gmask) HIPCHK(hipMemcpyAsync(E->d_batch, &B, sizeof(MsBatch), hipMemcpyHostToDevice, s));
   if (gmask)
     HIPCHK(scs_launch_ms_gdist(n, G, E->d_vis, gmask, E->d_dist16, E->d_batch, E->d_prepbytes, s));
+  const u64 packed = valid;  // before any query is sent back for want of room
   if (valid) {
-    HIPCHK(scs_launch_ms_scatter(n, G, E->d_vis, valid, E->d_gcnt, E->g->d_core, E->d_dist16,
+    HIPCHK(scs_launch_ms_scatter(n, G, E->d_vis, valid, E->d_gcnt, E->d_cbase, E->g->d_core, E->d_dist16,
                                  E->d_batch, E->d_locid64, E->d_tot + 128, E->d_prepbytes, s));
     HIPCHK(scs_launch_ms_degree(adj, E->d_units, E->nunits, E->d_hubs, E->nhubs, E->d_vis,
                                 valid, E->d_locid64, E->d_batch, E->d_hubcnt, E->d_prepbytes, s));
@@ -1035,12 +1042,13 @@ static int prep_batch(scs_engine* E, const u32* sis, const u32* kl0s, const u32*
         continue;
       }
       hs.b_len = b_len;
+      hs.nnz = nnz;
       B.P[b].ladj = (u32*)(E->d_arena + hs.b_off);
     }
     if (valid) {
       HIPCHK(hipMemcpyAsync(E->d_batch, &B, sizeof(MsBatch), hipMemcpyHostToDevice, s));
-      HIPCHK(scs_launch_ms_fill(adj, E->d_units, E->nunits, E->d_vis, valid, E->d_locid64,
-                                E->d_batch, E->d_hubcnt, E->d_prepbytes, s));
+      HIPCHK(scs_launch_ms_fill(adj, E->d_units, E->nunits, E->d_vis, valid, packed,
+                                E->d_locid64, E->d_batch, E->d_hubcnt, E->d_prepbytes, s));
     }
   }
   HIPCHK(hipEventRecord(E->pe1, s));
@@ -1485,9 +1493,7 @@ extern "C" int scs_prep_probe_many(scs_engine* E, uint32_t count, const uint32_t
     if (hs.whole) continue;  // no local graph (nnz stays 0)
     const QuerySlot& Q = E->h_slots[sis[i]];
     const u32 k = hs.K;
-    u32 nz = 0;
-    HIPCHK(hipMemcpy(&nz, Q.off + k, sizeof(u32), hipMemcpyDeviceToHost));
-    nnz[i] = nz;
+    nnz[i] = hs.nnz;
     if (k <= kept_cap) {
       if (kept)
         HIPCHK(hipMemcpy(kept + (u64)i * kept_cap, Q.orig, sizeof(u32) * k, hipMemcpyDeviceToHost));
@@ -1497,8 +1503,8 @@ extern "C" int scs_prep_probe_many(scs_engine* E, uint32_t count, const uint32_t
       if (dist)
         HIPCHK(hipMemcpy(dist + (u64)i * kept_cap, Q.dist, sizeof(u32) * k, hipMemcpyDeviceToHost));
     }
-    if (ladj && nz <= adj_cap)
-      HIPCHK(hipMemcpy(ladj + (u64)i * adj_cap, Q.adj, sizeof(u32) * (u64)nz,
+    if (ladj && hs.nnz <= adj_cap)
+      HIPCHK(hipMemcpy(ladj + (u64)i * adj_cap, Q.adj, sizeof(u32) * (u64)hs.nnz,
                        hipMemcpyDeviceToHost));
   }
   for (u32 si : sis) release_slot(E, si);

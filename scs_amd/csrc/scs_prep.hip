@@ -10,8 +10,10 @@
 //   elig[v]  queries whose BFS may enter v (core[v] > kl0_b).  The host
 //            numbers the queries by ascending kl0, so elig[v] is the mask of
 //            the first cnt(v) bits: one compare per query, no table.
-//   vis[v]   queries whose BFS reached v (= v is kept for them).
-//   fr / nf  queries for which v is in the current / next frontier.
+//   vis[v]   queries whose BFS reached v (= v is kept for them); a level's
+//            finds join it when the next level, or ms_count, reads them.
+//   fr / nf  queries for which v is in the current / next frontier (three
+//            buffers in turn: the third is cleared for the level after).
 // Level 0 pushes from the query vertices (top-down).  Every later level is
 // bottom-up (pull): every vertex that some active query still wants ORs the
 // frontier masks of its neighbours, stopping once it has every bit it
@@ -101,6 +103,11 @@ __device__ __forceinline__ u32 ms_wave_incl(u32 x) {
   }
   return x;
 }
+__device__ __forceinline__ u64 ms_uniform64(u64 x) {
+  // readfirstlane is signed: the low word must not spread its top bit
+  return ((u64)(u32)__builtin_amdgcn_readfirstlane((u32)(x >> 32)) << 32) |
+         (u32)__builtin_amdgcn_readfirstlane((u32)x);
+}
 // The wave number as a wave-uniform value.
 __device__ __forceinline__ u32 ms_wave_id() {
   return __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
@@ -111,7 +118,8 @@ __global__ void __launch_bounds__(256) ms_init(u32 n, const u32* __restrict__ co
                                                const MsBatch* __restrict__ B,
                                                u64* __restrict__ elig, u64* __restrict__ vis,
                                                u64* __restrict__ fr, u64* __restrict__ nf,
-                                               u32* __restrict__ flags, u32 nflags,
+                                               u64* __restrict__ xf, u32* __restrict__ flags,
+                                               u32 nflags,
                                                unsigned long long* bytes) {
   const u32 tid = blockIdx.x * blockDim.x + threadIdx.x;
   const u32 nt = gridDim.x * blockDim.x;
@@ -125,7 +133,8 @@ __global__ void __launch_bounds__(256) ms_init(u32 n, const u32* __restrict__ co
     vis[v] = 0;
     fr[v] = 0;
     nf[v] = 0;
-    nb += 4 + 32;
+    xf[v] = 0;
+    nb += 4 + 40;
   }
   for (u32 i = tid; i < nflags; i += nt) flags[i] = 0;
   ms_count_bytes(bytes, nb);
@@ -181,10 +190,18 @@ __global__ void __launch_bounds__(64) ms_push0(const i64* __restrict__ off,
 
 // One BFS level for every query whose depth bound exceeds `level` (act).
 // Runs only if the previous level found something (flag_prev).  A 16-lane
-// segment takes one vertex (four per wave) and reads 64 adjacency entries
-// per step, stopping once it holds every bit it wants; vertices of degree
-// above MS_HUB are taken by the whole wave, 512 entries per step.
-#define MS_HUB 512
+// segment takes one adjacency unit (at most MS_UNIT entries; four units per
+// wave) and reads 64 entries per step, stopping once it holds every bit it
+// wants.  A hub's units are spread over waves; each ORs what it found into nf,
+// which the level two before this one cleared for the hubs.  vis takes in the
+// current frontier here (vis | fr is the same whichever unit of a hub wrote
+// it), so no unit depends on another's finds of this level.
+//
+// Bound: the frontier gathers (8 bytes from a 64-byte line each, 16M of them
+// on the 500,000-vertex graph), and on hub-heavy graphs the longest wave: with
+// whole vertices per segment, and ids dealt out modulo the waves, an R-MAT
+// graph's hubs (ids with few bits set) met in one wave, and its second level
+// took 424 us where the 500,000-vertex graph's took 255; both take under 120 now (36 and 119).
 
 __device__ __forceinline__ u64 ms_seg_or(u64 x) {
   u32 lo = (u32)x, hi = (u32)(x >> 32);
@@ -194,12 +211,25 @@ __device__ __forceinline__ u64 ms_seg_or(u64 x) {
   }
   return ((u64)hi << 32) | lo;
 }
+// The bits of a find to the distance row of v, by the segment's lanes.
+__device__ __forceinline__ void ms_seg_dist(u16* __restrict__ dist16, u32 v, u64 acc, u32 level) {
+  for (u32 b = threadIdx.x & 15; b < 64; b += 16)
+    if ((acc >> b) & 1ull) dist16[(u64)v * MS_BITS + b] = (u16)(level + 1);
+}
+// Sets the level flag once: later waves read it from the L2 and skip the
+// atomic, so the finders do not queue on one address.
+__device__ __forceinline__ void ms_set_flag(u32* flag, bool found) {
+  if (__ballot(found) && (threadIdx.x & 63) == 0 &&
+      __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+    atomicOr(flag, 1u);
+}
 
-__global__ void __launch_bounds__(256) ms_level(const i64* __restrict__ off,
-                                                const int32_t* __restrict__ adj, u32 n, u32 level,
-                                                u64 act, const u64* __restrict__ elig,
-                                                u64* __restrict__ vis, const u64* __restrict__ fr,
-                                                u64* __restrict__ nf, u16* __restrict__ dist16,
+__global__ void __launch_bounds__(256) ms_level(const int32_t* __restrict__ adj,
+                                                const MsUnit* __restrict__ units, u32 nunits,
+                                                const MsHub* __restrict__ hubs, u32 nhubs,
+                                                u32 level, u64 act, const u64* __restrict__ elig,
+                                                u64* vis, const u64* fr, u64* nf, u64* clr,
+                                                u16* __restrict__ dist16,
                                                 const u32* __restrict__ flag_prev,
                                                 u32* __restrict__ flag_cur,
                                                 unsigned long long* bytes) {
@@ -207,43 +237,40 @@ __global__ void __launch_bounds__(256) ms_level(const i64* __restrict__ off,
   const u32 lane = threadIdx.x & 63, seg = lane >> 4, sl = lane & 15;
   const u64 wid = ms_wave_id();
   const u64 nw = ((u64)gridDim.x * blockDim.x) >> 6;
+  for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < nhubs; i += gridDim.x * blockDim.x)
+    clr[hubs[i].u] = 0;
   u64 nbytes = 0;
   bool found = false;
-  // segment s of wave w takes vertex (4*it + s)*nw + w at step it:
-  // neighbouring ids go to different waves, so a run of hubs (generators
-  // often number them first) is spread over the grid, not queued in one wave
-  for (u64 it = 0; it * 4 * nw < n; it++) {
-    const u64 vv = (4 * it + seg) * nw + wid;
-    const bool in = vv < n;
-    const u32 v = (u32)vv;
-    u64 want = 0, visv = 0;
-    i64 b0 = 0, e0 = 0;
-    if (in) {
-      visv = vis[v];
-      want = elig[v] & act & ~visv;
-      if (sl == 0) nbytes += 16;
+  for (u64 k0 = wid * 4; k0 < nunits; k0 += nw * 4) {
+    const bool in = k0 + seg < nunits;
+    const MsUnit U = units[in ? k0 + seg : nunits - 1];
+    const u32 v = U.u, len = (u32)(U.pos >> 48);
+    const i64 b0 = (i64)(U.pos & 0xFFFFFFFFFFFFull);
+    const u64 visv = vis[v], frv = fr[v], seen = visv | frv;
+    const u64 want = in ? elig[v] & act & ~seen : 0ull;
+    if (in && sl == 0) {
+      nbytes += 16 + 24;
+      if (frv & ~visv) {
+        vis[v] = seen;
+        nbytes += 8;
+      }
     }
-    if (want) {
-      b0 = off[v];
-      e0 = off[v + 1];
-      if (sl == 0) nbytes += 16;
-    }
-    const bool big = want && (e0 - b0) > MS_HUB;
-    bool active = want && !big;
     // 64 entries per segment step: each lane issues its four adjacency
     // loads, then its four frontier gathers, so a step costs two memory
     // round trips
     u64 acc = 0;
-    i64 j = b0 + sl;
+    u32 j = sl;
+    bool active = want != 0 && len != 0;
     while (__ballot(active)) {
       u64 x = 0;
       if (active) {
         u32 w[4];
 #pragma unroll
-        for (int t = 0; t < 4; t++) w[t] = j + 16 * t < e0 ? (u32)adj[j + 16 * t] : 0u;
+        for (int t = 0; t < 4; t++)
+          w[t] = j + 16 * t < len ? (u32)__builtin_nontemporal_load(&adj[b0 + j + 16 * t]) : v;
 #pragma unroll
         for (int t = 0; t < 4; t++)
-          if (j + 16 * t < e0) {
+          if (j + 16 * t < len) {
             x |= fr[w[t]];
             nbytes += 12;
           }
@@ -251,109 +278,112 @@ __global__ void __launch_bounds__(256) ms_level(const i64* __restrict__ off,
       }
       acc |= ms_seg_or(x);
       j += 64;
-      if (active && (acc == want || j - (i64)sl >= e0)) active = false;
-    }
-    // hubs: the whole wave, 512 entries per step
-    u64 bm = __ballot(big && sl == 0);
-    while (bm) {
-      const int src = __ffsll((unsigned long long)bm) - 1;
-      bm &= bm - 1;
-      const u64 bwant = ms_shfl64(want, src);
-      const i64 bb = (i64)ms_shfl64((u64)b0, src), be = (i64)ms_shfl64((u64)e0, src);
-      u64 bacc = 0;
-      for (i64 jj = bb + lane; jj - (i64)lane < be; jj += 512) {
-        u32 w[8];
-#pragma unroll
-        for (int t = 0; t < 8; t++) w[t] = jj + 64 * t < be ? (u32)adj[jj + 64 * t] : 0u;
-        u64 x = 0;
-#pragma unroll
-        for (int t = 0; t < 8; t++)
-          if (jj + 64 * t < be) {
-            x |= fr[w[t]];
-            nbytes += 12;
-          }
-        bacc |= ms_or(x & bwant);
-        if (bacc == bwant) break;
-      }
-      // hand the result to the hub's segment
-      if ((lane >> 4) == ((u32)src >> 4)) acc = bacc;
+      if (active && (acc == want || j - sl >= len)) active = false;
     }
     if (in) {
-      if (sl == 0) {
-        nf[v] = acc;
+      if (U.h == MS_NOHUB) {
+        if (sl == 0) {
+          nf[v] = acc;
+          nbytes += 8;
+        }
+      } else if (acc && sl == 0) {
+        atomicOr((unsigned long long*)&nf[v], (unsigned long long)acc);
         nbytes += 8;
       }
       if (acc) {
-        if (sl == 0) {
-          vis[v] = visv | acc;
-          nbytes += 8;
-        }
         found = true;
-        for (u32 b = sl; b < 64; b += 16)
-          if ((acc >> b) & 1ull) {
-            dist16[(u64)v * MS_BITS + b] = (u16)(level + 1);
-            nbytes += 2;
-          }
+        ms_seg_dist(dist16, v, acc, level);
+        if (sl == 0) nbytes += 2ull * (u32)__popcll(acc);
       }
     }
   }
-  // set the level flag once: later waves read it from the L2 and skip the
-  // atomic, so the finders do not queue on one address
-  if (__ballot(found) && lane == 0 &&
-      __hip_atomic_load(flag_cur, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-    atomicOr(flag_cur, 1u);
+  ms_set_flag(flag_cur, found);
   ms_count_bytes(bytes, nbytes);
 }
 
-// Per 64-vertex group g and query b: number of group vertices kept by b,
-// stored at gcnt[g * 64 + b].
-__global__ void __launch_bounds__(256) ms_count(u32 n, u32 G, const u64* __restrict__ vis,
-                                                u64 valid, u32* __restrict__ gcnt,
+// Kept counts.  A wave takes MS_CHUNK groups of 64 vertices, lane b counting
+// for query b: gcnt[g * 64 + b] = query b's kept vertices in the chunk's groups
+// before g, cbase[c * 64 + b] = those in chunk c.  vis takes in the last
+// level's finds (lf; bits already there when the search ended earlier).
+#define MS_CHUNK 32
+__global__ void __launch_bounds__(256) ms_count(u32 n, u32 G, u64* __restrict__ vis,
+                                                const u64* __restrict__ lf, u64 valid,
+                                                u32* __restrict__ gcnt, u32* __restrict__ cbase,
                                                 unsigned long long* bytes) {
   const u32 lane = threadIdx.x & 63;
-  const u32 wid = ms_wave_id();
-  const u32 nw = (gridDim.x * blockDim.x) >> 6;
+  const u32 c = ms_wave_id();
+  const u32 g0 = c * MS_CHUNK;
+  if (g0 >= G) return;
+  const u32 g1 = min(G, g0 + MS_CHUNK);
   u64 nbytes = 0;
-  for (u32 g = wid; g < G; g += nw) {
-    const u64 v = (u64)g * 64 + lane;
-    const u64 m = v < n ? vis[v] & valid : 0;
-    if (v < n) nbytes += 8;
-    // lane b: the group's vertices kept by query b
-    gcnt[(u64)g * 64 + lane] = (u32)__popcll(ms_transpose(m));
-    nbytes += 4;
+  u32 run = 0;
+  for (u32 g = g0; g < g1; g += 8) {
+    u64 m[8], f[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+      const u64 v = (u64)(g + t) * 64 + lane;
+      const bool in = g + t < g1 && v < n;
+      m[t] = in ? vis[v] : 0ull;
+      f[t] = in ? lf[v] : 0ull;
+    }
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+      if (g + t >= g1) break;
+      const u64 v = (u64)(g + t) * 64 + lane;
+      if (f[t] & ~m[t]) vis[v] = m[t] | f[t];
+      if (v < n) nbytes += 16;
+      gcnt[(u64)(g + t) * 64 + lane] = run;
+      run += (u32)__popcll(ms_transpose((m[t] | f[t]) & valid));
+      nbytes += 4;
+    }
   }
-  ms_count_bytes(bytes, nbytes);
+  cbase[(u64)c * 64 + lane] = run;
+  ms_count_bytes(bytes, nbytes + 4);
 }
 
-// One workgroup per query b: group counts -> exclusive bases in place;
-// K_b -> tot[b].
-// One wave per query and no LDS, so the pass also finds room on CUs whose
-// LDS the search kernel holds.
-__global__ void __launch_bounds__(64) ms_bscan(u32 G, u32* __restrict__ gcnt, u32* __restrict__ tot,
-                                               unsigned long long* bytes) {
-  const u32 b = blockIdx.x, t = threadIdx.x;
-  const u32 per = (G + 63) / 64;
-  const u32 g0 = min(G, t * per), g1 = min(G, g0 + per);
-  u32 s = 0;
-  for (u32 g = g0; g < g1; g++) s += gcnt[(u64)g * 64 + b];
-  const u32 incl = ms_wave_incl(s);
-  u32 run = incl - s;
-  for (u32 g = g0; g < g1; g++) {
-    const u32 c = gcnt[(u64)g * 64 + b];
-    gcnt[(u64)g * 64 + b] = run;
-    run += c;
+// Chunk counts -> exclusive bases in place; K_b -> tot[b].  One wave, lane =
+// query, eight coalesced rows in flight.  (One wave per query over the
+// group counts, 256 bytes apart per lane, took 62 us on 500,000 vertices;
+// counting by chunks first leaves 245 rows.)
+__global__ void __launch_bounds__(64) ms_bscan(u32 C, u32* __restrict__ cbase,
+                                               u32* __restrict__ tot, unsigned long long* bytes) {
+  const u32 b = threadIdx.x;
+  u32 run = 0;
+  for (u32 c = 0; c < C; c += 8) {
+    u32 x[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) x[t] = cbase[(u64)min(c + t, C - 1) * 64 + b];
+#pragma unroll
+    for (int t = 0; t < 8; t++)
+      if (c + t < C) {
+        cbase[(u64)(c + t) * 64 + b] = run;
+        run += x[t];
+      }
   }
-  if (t == 63) tot[b] = incl;
-  ms_count_bytes(bytes, (u64)(g1 - g0) * 12);
+  tot[b] = run;
+  ms_count_bytes(bytes, (u64)C * 8 + 4);
 }
+
+// Columns of the local-id rows (locid, one row per vertex): the groups of
+// eight queries that the pass takes, packed, so that a batch which leaves few
+// queries to it has rows of 8 or 16 entries instead of 64, whose gathers the
+// caches can hold (500,000 vertices: 16 MB instead of 128).
+struct MsCols {
+  u32 rank;    // 4 bits per group of eight queries: its place in a row
+  u32 stride;  // entries per row
+  __device__ __forceinline__ u32 group(u32 g) const { return ((rank >> (4 * g)) & 15u) * 8; }
+  __device__ __forceinline__ u32 col(u32 b) const { return group(b >> 3) + (b & 7); }
+};
 
 // Local ids, and per kept vertex: orig id, distance, core number.
 __global__ void __launch_bounds__(256) ms_scatter(u32 n, u32 G, const u64* __restrict__ vis,
                                                   u64 valid, const u32* __restrict__ gcnt,
+                                                  const u32* __restrict__ cbase,
                                                   const u32* __restrict__ core,
                                                   const u16* __restrict__ dist16,
                                                   const MsBatch* __restrict__ B,
-                                                  u32* __restrict__ locid, u32* __restrict__ qloc,
+                                                  u32* __restrict__ locid, MsCols cols,
+                                                  u32* __restrict__ qloc,
                                                   unsigned long long* bytes) {
   const u32 lane = threadIdx.x & 63;
   const u32 wid = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -367,7 +397,8 @@ __global__ void __launch_bounds__(256) ms_scatter(u32 n, u32 G, const u64* __res
   for (u32 g = wid; g < G; g += nw) {
     const u64 v = (u64)g * 64 + lane;
     const u64 m = v < n ? vis[v] & valid : 0;
-    const u32 gb = gcnt[(u64)g * 64 + lane];  // lane b: query b's first id in the group
+    // lane b: query b's first id in the group
+    const u32 gb = gcnt[(u64)g * 64 + lane] + cbase[(u64)(g / MS_CHUNK) * 64 + lane];
     u32 cv = 0;
     if (m) {
       cv = core[v];
@@ -401,7 +432,7 @@ __global__ void __launch_bounds__(256) ms_scatter(u32 n, u32 G, const u64* __res
           lorig[id] = (u32)v;
           ldist[id] = dv[t];
           lcore[id] = cv;
-          locid[v * MS_BITS + b] = id;
+          locid[v * cols.stride + cols.col(b)] = id;
           if ((u32)v == qv) qloc[b] = id;
           nbytes += 4 + 2 + 12 + 4;
         }
@@ -413,9 +444,11 @@ __global__ void __launch_bounds__(256) ms_scatter(u32 n, u32 G, const u64* __res
 
 // Whole-graph queries (gmask): query b's distance array over every vertex of
 // the graph, SCS_DIST_NONE where b does not keep the vertex.  Lane = vertex,
-// so each query's 64 values of a group are one coalesced store.  Queries are
-// taken eight at a time: their eight distance loads are in flight together
-// before the eight stores.
+// so each query's 64 values of a group are one coalesced store; a lane reads
+// its vertex's row of 64 distances as eight 16-byte loads, all in flight, so a
+// row's line is fetched once.  Bound: stores (4 bytes per query and vertex).
+// 500,000 vertices, 59 such queries: 41 us; one 2-byte load per query and
+// vertex, eight queries at a time, took 102.
 __global__ void __launch_bounds__(256) ms_gdist(u32 n, u32 G, const u64* __restrict__ vis,
                                                 u64 gmask, const u16* __restrict__ dist16,
                                                 const MsBatch* __restrict__ B,
@@ -428,99 +461,112 @@ __global__ void __launch_bounds__(256) ms_gdist(u32 n, u32 G, const u64* __restr
   for (u32 g = wid; g < G; g += nw) {
     const u64 v = (u64)g * 64 + lane;
     const bool in = v < n;
-    const u64 m = in ? vis[v] & gmask : 0ull;
-    if (in) nbytes += 8;
-    u64 left = gmask;
-    while (left) {
-      int bb[8];
-      u32 dv[8];
+    const u64 vv = in ? v : (u64)n - 1;
+    const u64 m = in ? vis[vv] & gmask : 0ull;
+    uint4 d[8];
 #pragma unroll
-      for (int t = 0; t < 8; t++) {
-        bb[t] = left ? __ffsll((unsigned long long)left) - 1 : -1;
-        left &= left - 1;  // 0 stays 0
-      }
+    for (int t = 0; t < 8; t++)
+      if ((gmask >> (8 * t)) & 0xFFull) d[t] = *(const uint4*)&dist16[vv * MS_BITS + 8 * t];
+    if (in) nbytes += 8 + 4ull * (u32)__popcll(gmask) + 2ull * (u32)__popcll(m);
 #pragma unroll
-      for (int t = 0; t < 8; t++) {
-        const bool kept = bb[t] >= 0 && ((m >> bb[t]) & 1ull);
-        dv[t] = kept ? (u32)dist16[v * MS_BITS + bb[t]] : SCS_DIST_NONE;
-        if (in && bb[t] >= 0) nbytes += kept ? 6 : 4;
-      }
+    for (int t = 0; t < 8; t++) {
+      const u32 x[4] = {d[t].x, d[t].y, d[t].z, d[t].w};
 #pragma unroll
-      for (int t = 0; t < 8; t++) {
-        if (bb[t] < 0) break;
-        u32* const d = (u32*)ms_shfl64(dp, bb[t]);
-        if (in) d[v] = dv[t];
+      for (int i = 0; i < 8; i++) {
+        const int b = 8 * t + i;
+        if (!((gmask >> b) & 1ull)) continue;
+        const u32 dv = (x[i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
+        u32* const o = (u32*)ms_shfl64(dp, b);
+        if (in) o[v] = (m >> b) & 1ull ? dv : SCS_DIST_NONE;
       }
     }
   }
   ms_count_bytes(bytes, nbytes);
 }
 
-// One adjacency unit (at most MS_UNIT entries): lane i loads entries i,
-// i+64, i+128, i+192, then their vis words, and keeps w[t] = the neighbour
-// id (0 past the unit's end) and mw[t] = the queries that keep that
-// neighbour.  (Unconditional loads from clamped indices, which let all
-// eight be in flight, measured no faster: most units have one chunk.)
-__device__ __forceinline__ void ms_unit_load(const int32_t* __restrict__ adj,
-                                             const u64* __restrict__ vis, i64 b0, u32 len,
-                                             u32 w[4], u64 mw[4], u64& nbytes) {
+// One adjacency unit (at most MS_UNIT entries) as the local degree and
+// adjacency passes take it: lane i holds entries i, i+64, i+128, i+192 (0 past
+// the unit's end), lane b query b's local id of the unit's vertex.  A wave
+// loads the next unit while it works on this one, so a unit costs two round
+// trips less than its chain of header, entries, keep masks and rows; the keep
+// masks of the entries, gathers all over the graph, are read only for a vertex
+// that some query of the pass keeps.
+struct MsUnitRegs {
+  u32 u, h, len, id, w[4];
+  u64 mu;  // the pass's queries that keep u
+};
+__device__ __forceinline__ void ms_unit_load(const int32_t* __restrict__ adj, const MsUnit& U,
+                                             const u64* __restrict__ vis, u64 valid,
+                                             const u32* __restrict__ locid, const MsCols& cols,
+                                             MsUnitRegs& R) {
   const u32 lane = threadIdx.x & 63;
+  const i64 b0 = (i64)(U.pos & 0xFFFFFFFFFFFFull);
+  R.u = U.u;
+  R.h = U.h;
+  R.len = (u32)(U.pos >> 48);
+  R.mu = vis[U.u] & valid;
+  R.id = locid[(u64)U.u * cols.stride + cols.col(lane)];
 #pragma unroll
-  for (int t = 0; t < 4; t++) w[t] = lane + 64u * t < len ? (u32)adj[b0 + lane + 64 * t] : 0u;
+  for (int t = 0; t < 4; t++) R.w[t] = lane + 64u * t < R.len ? (u32)adj[b0 + lane + 64 * t] : 0u;
+}
+// mw[t] = the queries that keep entry t.
+__device__ __forceinline__ void ms_unit_masks(const u64* __restrict__ vis, const MsUnitRegs& R,
+                                              u64 mw[4], u64& nbytes) {
+  const u32 lane = threadIdx.x & 63;
 #pragma unroll
   for (int t = 0; t < 4; t++) {
     mw[t] = 0;
-    if (lane + 64u * t < len) {
-      mw[t] = vis[w[t]];
+    if (lane + 64u * t < R.len) {
+      mw[t] = vis[R.w[t]];
       nbytes += 12;
     }
   }
 }
-__device__ __forceinline__ i64 ms_unit_b0(const MsUnit& U) {
-  return (i64)(U.pos & 0xFFFFFFFFFFFFull);
-}
-__device__ __forceinline__ u32 ms_unit_len(const MsUnit& U) { return (u32)(U.pos >> 48); }
 
 // Local degree of every (query, kept vertex).  One wave per adjacency unit;
 // lane b counts query b's kept neighbours in the unit as the popcount of
 // column b of the transposed keep masks.  A single-unit vertex writes
 // loff[id] directly; a hub's units write partial counts to hubcnt, which
-// ms_hubsum turns into unit offsets and the degree.  The unit's vis word,
-// locid row and adjacency are loaded together, before the keep test.
+// ms_hubsum turns into unit offsets and the degree.
+// Bound: round trips.  500,000 vertices, 16M entries, 5 queries: 137 us, 164 with
+// one unit at a time.
 __global__ void __launch_bounds__(256) ms_degree(const int32_t* __restrict__ adj,
                                                  const MsUnit* __restrict__ units, u32 nunits,
                                                  const u64* __restrict__ vis, u64 valid,
-                                                 const u32* __restrict__ locid,
+                                                 const u32* __restrict__ locid, MsCols cols,
                                                  const MsBatch* __restrict__ B,
                                                  u32* __restrict__ hubcnt,
                                                  unsigned long long* bytes) {
   const u32 lane = threadIdx.x & 63;
   const u32 wid = ms_wave_id();
   const u32 nw = (gridDim.x * blockDim.x) >> 6;
+  if (wid >= nunits) return;
   u32* const loff = B->P[lane].loff;
   u64 nbytes = 0;
-  for (u32 k = wid; k < nunits; k += nw) {
-    const MsUnit U = units[k];
-    const i64 b0 = ms_unit_b0(U);
-    const u32 len = ms_unit_len(U);
-    const u64 mu = vis[U.u] & valid;
-    const u32 id = locid[(u64)U.u * MS_BITS + lane];
-    u32 w[4] = {0u, 0u, 0u, 0u};
-    u64 mw[4] = {0ull, 0ull, 0ull, 0ull};
-    if (len) ms_unit_load(adj, vis, b0, len, w, mw, nbytes);
+  MsUnitRegs N;
+  ms_unit_load(adj, units[wid], vis, valid, locid, cols, N);
+  MsUnit Un = units[(u64)wid + nw < nunits ? wid + nw : wid];
+  for (u64 k = wid; k < nunits; k += nw) {
+    const MsUnitRegs R = N;
+    if (k + nw < nunits) {
+      ms_unit_load(adj, Un, vis, valid, locid, cols, N);
+      if (k + 2ull * nw < nunits) Un = units[k + 2ull * nw];
+    }
     if (lane == 0) nbytes += 16 + 8;
-    if (!mu) continue;
+    if (!R.mu) continue;
+    u64 mw[4];
+    ms_unit_masks(vis, R, mw, nbytes);
     u32 cnt = 0;
 #pragma unroll
     for (int t = 0; t < 4; t++)
-      if (64u * t < len) cnt += (u32)__popcll(ms_transpose(mw[t] & mu));
-    if (U.h == MS_NOHUB) {
-      if ((mu >> lane) & 1ull) {
-        loff[id] = cnt;
+      if (64u * t < R.len) cnt += (u32)__popcll(ms_transpose(mw[t] & R.mu));
+    if (R.h == MS_NOHUB) {
+      if ((R.mu >> lane) & 1ull) {
+        loff[R.id] = cnt;
         nbytes += 8;
       }
     } else {
-      hubcnt[(u64)U.h * 64 + lane] = cnt;
+      hubcnt[(u64)R.h * 64 + lane] = cnt;
       nbytes += 4;
     }
   }
@@ -531,7 +577,7 @@ __global__ void __launch_bounds__(256) ms_degree(const int32_t* __restrict__ adj
 // exclusive unit offsets (in place) and writes the degree to loff[id].
 __global__ void __launch_bounds__(256) ms_hubsum(const MsHub* __restrict__ hubs, u32 nhubs,
                                                  const u64* __restrict__ vis, u64 valid,
-                                                 const u32* __restrict__ locid,
+                                                 const u32* __restrict__ locid, MsCols cols,
                                                  const MsBatch* __restrict__ B,
                                                  u32* __restrict__ hubcnt,
                                                  unsigned long long* bytes) {
@@ -553,7 +599,7 @@ __global__ void __launch_bounds__(256) ms_hubsum(const MsHub* __restrict__ hubs,
     }
     nbytes += (u64)H.nu * 8;
     if ((mu >> lane) & 1ull) {
-      const u32 id = locid[(u64)H.u * MS_BITS + lane];
+      const u32 id = locid[(u64)H.u * cols.stride + cols.col(lane)];
       B->P[lane].loff[id] = run;
       nbytes += 8;
     }
@@ -685,92 +731,100 @@ __global__ void __launch_bounds__(256) ms_loff_apply(const MsBatch* __restrict__
 // One wave per adjacency unit.  Query b's entries of the unit go to its
 // write position dst_b, in neighbour order; column b of the transposed keep
 // masks says which neighbours query b keeps.  The work is cut into tiles of
-// MS_FILL_QT queries x (64 / MS_FILL_QT) neighbours: lane (ji, qi) =
-// (lane / QT, lane % QT) takes query qb*QT+qi and neighbour jb*JT+ji.  A
-// store instruction then writes QT runs of up to JT consecutive entries and
-// a load instruction reads JT pieces of QT entries of the locid rows, where
-// a whole-row or whole-column form touches 64 lines with one of the two.
-// On C2 (Chung-Lu, 100K vertices) 8 x 8 tiles with 32 row loads in flight
-// were fastest; 4 x 16 and 2 x 32 were 1 % and 22 % slower, non-temporal
-// stores (no write-combining in the L2) 2.7x slower, and runs of 2 to 8
-// consecutive units per wave 3-6 % slower.
-#ifndef MS_FILL_QT
-#define MS_FILL_QT 8
-#endif
-#ifndef MS_FILL_LOADS
-#define MS_FILL_LOADS 32  // row loads in flight per wave
-#endif
-__global__ void __launch_bounds__(256) ms_fill(const int32_t* __restrict__ adj,
+// 8 queries x 8 neighbours: lane (ji, qi) = (lane / 8, lane % 8) takes query
+// 8 qb + qi and neighbour 8 jb + ji.  A store instruction then writes eight
+// runs of up to eight consecutive entries and a load instruction reads eight
+// pieces of eight entries of the locid rows, where a whole-row or whole-column
+// form touches 64 lines with one of the two.
+//
+// FEW: one group of eight queries at a time, for batches that leave at most
+// MS_FILL_FEW queries to this pass: groups without a query that keeps the
+// vertex and tiles past the unit's end are passed over, and the registers that
+// saves let twice the waves hide the round trips.  Else four groups at a time,
+// with all their 32 row loads in flight and no branches between them.
+// 500,000 vertices, 5 queries: 354 us, 525 before; 131,072 (R-MAT), 35 queries:
+// 314, 312 before.
+// Ids from per-group keep bits (16 bytes per query and 64 vertices) in place
+// of the rows were 1.5 times slower; non-temporal stores 2.7 times.
+#define MS_FILL_FEW 16
+template <bool FEW>
+__global__ void __launch_bounds__(256, FEW ? 6 : 1) ms_fill(const int32_t* __restrict__ adj,
                                                const MsUnit* __restrict__ units, u32 nunits,
                                                const u64* __restrict__ vis, u64 valid,
-                                               const u32* __restrict__ locid,
+                                               const u32* __restrict__ locid, MsCols cols,
                                                const MsBatch* __restrict__ B,
                                                const u32* __restrict__ hubcnt,
                                                unsigned long long* bytes) {
-  constexpr u32 QT = MS_FILL_QT, JT = 64 / QT, QG = MS_FILL_LOADS / QT;
-  constexpr u64 GMASK = QG * QT == 64 ? ~0ull : ((1ull << (QG * QT)) - 1ull);
-  constexpr u64 JMASK = JT == 64 ? ~0ull : ((1ull << JT) - 1ull);
+  constexpr u32 QG = FEW ? 1 : 4;
+  constexpr u64 GMASK = (1ull << (QG * 8)) - 1ull;
   const u32 lane = threadIdx.x & 63;
   const u32 wid = ms_wave_id();
   const u32 nw = (gridDim.x * blockDim.x) >> 6;
-  const u32 qi = lane % QT, ji = lane / QT;
-  const u64 below = ji ? (~0ull >> (64 - ji)) : 0ull;
+  if (wid >= nunits) return;
+  const u32 qi = lane % 8, ji = lane / 8;
+  const u32 below = (1u << ji) - 1u;
   const u32* const loff = B->P[lane].loff;
   u32* const ladj = B->P[lane].ladj;
   u64 nbytes = 0;
-  for (u32 k = wid; k < nunits; k += nw) {
-    const MsUnit U = units[k];
-    const i64 b0 = ms_unit_b0(U);
-    const u32 len = ms_unit_len(U);
-    const u64 mu = vis[U.u] & valid;
-    const u32 id = locid[(u64)U.u * MS_BITS + lane];
-    const u32 part = hubcnt[(U.h != MS_NOHUB ? (u64)U.h * 64 : 0ull) + lane] &
-                     (U.h != MS_NOHUB ? ~0u : 0u);
-    u32 w[4] = {0u, 0u, 0u, 0u};
-    u64 mw[4] = {0ull, 0ull, 0ull, 0ull};
-    if (len) ms_unit_load(adj, vis, b0, len, w, mw, nbytes);
+  MsUnitRegs N;
+  ms_unit_load(adj, units[wid], vis, valid, locid, cols, N);
+  MsUnit Un = units[(u64)wid + nw < nunits ? wid + nw : wid];
+  for (u64 k = wid; k < nunits; k += nw) {
+    const MsUnitRegs R = N;
+    if (k + nw < nunits) {
+      ms_unit_load(adj, Un, vis, valid, locid, cols, N);
+      if (k + 2ull * nw < nunits) Un = units[k + 2ull * nw];
+    }
     if (lane == 0) nbytes += 16 + 8;
+    const u64 mu = ms_uniform64(R.mu);
     if (!mu) continue;
+    const u32 len = __builtin_amdgcn_readfirstlane(R.len);
+    u64 mw[4];
+    ms_unit_masks(vis, R, mw, nbytes);
     // lane b: where query b's entries of this unit go
     u64 dst = 0;
     if ((mu >> lane) & 1ull) {
-      dst = (u64)(ladj + loff[id] + part);
+      const u32 part = R.h != MS_NOHUB ? hubcnt[(u64)R.h * 64 + lane] : 0u;
+      dst = (u64)(ladj + loff[R.id] + part);
       nbytes += 8;
     }
-    const u32 nt = (len + 63) / 64;
     u64 col[4];  // lane b: bit j = query b keeps entry 64t + j
 #pragma unroll
-    for (int t = 0; t < 4; t++) col[t] = (u32)t < nt ? ms_transpose(mw[t] & mu) : 0ull;
+    for (int t = 0; t < 4; t++) col[t] = 64u * t < len ? ms_transpose(mw[t] & mu) : 0ull;
 #pragma unroll
     for (int t = 0; t < 4; t++) nbytes += 8ull * (u32)__popcll(col[t]);
-    // QG query groups at a time, so QG * QT row loads are in flight
-    for (u32 qb0 = 0; qb0 < 64 / QT; qb0 += QG) {
-      if (!((mu >> (qb0 * QT)) & GMASK)) continue;  // none of these queries keeps U.u
+    for (u32 qb0 = 0; qb0 < 8; qb0 += QG) {
+      if (!((mu >> (qb0 * 8)) & GMASK)) continue;  // none of these queries keeps the vertex
       __attribute__((address_space(1))) u32* dq[QG];
 #pragma unroll
       for (u32 x = 0; x < QG; x++)
-        dq[x] = (__attribute__((address_space(1))) u32*)ms_shfl64(dst, (int)((qb0 + x) * QT + qi));
+        dq[x] = (__attribute__((address_space(1))) u32*)ms_shfl64(dst, (int)((qb0 + x) * 8 + qi));
 #pragma unroll
       for (int t = 0; t < 4; t++) {
-        if ((u32)t >= nt) break;
-        u32 wj[QT];  // w[t] is 0 past the unit's end, so every row index is a vertex
+        if (64u * t >= len) break;
+        const u32 nj = FEW ? (min(64u, len - 64u * t) + 7) / 8 : 8u;  // blocks to take
+        u32 wj[8];  // an entry is 0 past the unit's end, so every row index is a vertex
 #pragma unroll
-        for (u32 jb = 0; jb < QT; jb++) wj[jb] = (u32)__shfl(w[t], (int)(jb * JT + ji));
-        u32 r[QG][QT];
+        for (u32 jb = 0; jb < 8; jb++)
+          if (jb < nj) wj[jb] = (u32)__shfl(R.w[t], (int)(jb * 8 + ji));
+        u32 r[QG][8];
 #pragma unroll
         for (u32 x = 0; x < QG; x++)
 #pragma unroll
-          for (u32 jb = 0; jb < QT; jb++)
-            r[x][jb] = locid[(u64)wj[jb] * MS_BITS + (qb0 + x) * QT + qi];
+          for (u32 jb = 0; jb < 8; jb++)
+            if (jb < nj)
+              r[x][jb] = locid[(u64)wj[jb] * cols.stride + cols.group(qb0 + x) + qi];
 #pragma unroll
         for (u32 x = 0; x < QG; x++) {
-          const u64 colq = ms_shfl64(col[t], (int)((qb0 + x) * QT + qi));
+          const u32 clo = __shfl((u32)col[t], (int)((qb0 + x) * 8 + qi));
+          const u32 chi = __shfl((u32)(col[t] >> 32), (int)((qb0 + x) * 8 + qi));
 #pragma unroll
-          for (u32 jb = 0; jb < QT; jb++) {
-            const u64 bits = (colq >> (jb * JT)) & JMASK;
-            if ((bits >> ji) & 1ull) dq[x][__popcll(bits & below)] = r[x][jb];
-            dq[x] += __popcll(bits);
-          }
+          for (u32 jb = 0; jb < 8; jb++)
+            if (jb < nj) {
+              const u32 bits = ((jb < 4 ? clo : chi) >> (8 * (jb & 3))) & 0xFFu;
+              if ((bits >> ji) & 1u) dq[x][__popc(bits & below)] = r[x][jb];
+              dq[x] += __popc(bits);
+            }
         }
       }
     }
@@ -784,6 +838,15 @@ __global__ void __launch_bounds__(256) ms_fill(const int32_t* __restrict__ adj,
 // Grid-stride kernels launch at most one generation of resident waves
 // (2048 blocks of four waves = 8 waves on each SIMD of 256 CUs).
 #define MS_GRID 2048
+static MsCols ms_cols(u64 valid) {
+  MsCols c{0, 0};
+  for (u32 g = 0; g < 8; g++)
+    if ((valid >> (8 * g)) & 0xFFull) {
+      c.rank |= (c.stride / 8) << (4 * g);
+      c.stride += 8;
+    }
+  return c;
+}
 static u32 ms_blocks(u64 threads, u32 cap) {
   u64 b = (threads + 255) / 256;
   if (b == 0) b = 1;
@@ -791,9 +854,9 @@ static u32 ms_blocks(u64 threads, u32 cap) {
 }
 
 extern "C" hipError_t scs_launch_ms_init(u32 n, const u32* core, const MsBatch* B, u64* elig,
-                                         u64* vis, u64* fr, u64* nf, u32* flags, u32 nflags,
-                                         unsigned long long* bytes, hipStream_t s) {
-  ms_init<<<ms_blocks(n, MS_GRID), 256, 0, s>>>(n, core, B, elig, vis, fr, nf, flags, nflags,
+                                         u64* vis, u64* fr, u64* nf, u64* xf, u32* flags,
+                                         u32 nflags, unsigned long long* bytes, hipStream_t s) {
+  ms_init<<<ms_blocks(n, MS_GRID), 256, 0, s>>>(n, core, B, elig, vis, fr, nf, xf, flags, nflags,
                                                 bytes);
   return hipGetLastError();
 }
@@ -809,25 +872,30 @@ extern "C" hipError_t scs_launch_ms_seed(const MsBatch* B, u64* vis, u64* fr, u1
   ms_seed<<<1, 64, 0, s>>>(B, vis, fr, dist16);
   return hipGetLastError();
 }
-extern "C" hipError_t scs_launch_ms_level(const i64* off, const int32_t* adj, u32 n, u32 level,
-                                          u64 act, const u64* elig, u64* vis, const u64* fr,
-                                          u64* nf, u16* dist16, const u32* flag_prev,
+extern "C" hipError_t scs_launch_ms_level(const int32_t* adj, const MsUnit* units, u32 nunits,
+                                          const MsHub* hubs, u32 nhubs, u32 level, u64 act,
+                                          const u64* elig, u64* vis, const u64* fr, u64* nf,
+                                          u64* clr, u16* dist16, const u32* flag_prev,
                                           u32* flag_cur, unsigned long long* bytes,
                                           hipStream_t s) {
-  ms_level<<<ms_blocks(((u64)n + 3) / 4 * 64, MS_GRID), 256, 0, s>>>(
-      off, adj, n, level, act, elig, vis, fr, nf, dist16, flag_prev, flag_cur, bytes);
+  ms_level<<<ms_blocks(((u64)nunits + 3) / 4 * 64, MS_GRID), 256, 0, s>>>(
+      adj, units, nunits, hubs, nhubs, level, act, elig, vis, fr, nf, clr, dist16, flag_prev,
+      flag_cur, bytes);
   return hipGetLastError();
 }
-extern "C" hipError_t scs_launch_ms_count(u32 n, u32 G, const u64* vis, u64 valid, u32* gcnt,
+// Kept counts and their bases: gcnt holds G * 64 words, cbase one row of 64
+// per MS_CHUNK groups.
+extern "C" hipError_t scs_launch_ms_count(u32 n, u32 G, u64* vis, const u64* lf, u64 valid,
+                                          u32* gcnt, u32* cbase, u32* tot,
                                           unsigned long long* bytes, hipStream_t s) {
-  ms_count<<<ms_blocks((u64)G * 64, MS_GRID), 256, 0, s>>>(n, G, vis, valid, gcnt, bytes);
+  const u32 C = (G + MS_CHUNK - 1) / MS_CHUNK;
+  if (C) ms_count<<<(C + 3) / 4, 256, 0, s>>>(n, G, vis, lf, valid, gcnt, cbase, bytes);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  ms_bscan<<<1, 64, 0, s>>>(C, cbase, tot, bytes);
   return hipGetLastError();
 }
-extern "C" hipError_t scs_launch_ms_bscan(u32 nb, u32 G, u32* gcnt, u32* tot,
-                                          unsigned long long* bytes, hipStream_t s) {
-  ms_bscan<<<nb, 64, 0, s>>>(G, gcnt, tot, bytes);
-  return hipGetLastError();
-}
+extern "C" u64 scs_ms_count_rows(u32 G) { return (G + MS_CHUNK - 1) / MS_CHUNK; }
 extern "C" hipError_t scs_launch_ms_gdist(u32 n, u32 G, const u64* vis, u64 gmask,
                                           const u16* dist16, const MsBatch* B,
                                           unsigned long long* bytes, hipStream_t s) {
@@ -835,11 +903,12 @@ extern "C" hipError_t scs_launch_ms_gdist(u32 n, u32 G, const u64* vis, u64 gmas
   return hipGetLastError();
 }
 extern "C" hipError_t scs_launch_ms_scatter(u32 n, u32 G, const u64* vis, u64 valid,
-                                            const u32* gcnt, const u32* core, const u16* dist16,
+                                            const u32* gcnt, const u32* cbase, const u32* core,
+                                            const u16* dist16,
                                             const MsBatch* B, u32* locid, u32* qloc,
                                             unsigned long long* bytes, hipStream_t s) {
-  ms_scatter<<<ms_blocks((u64)G * 64, MS_GRID), 256, 0, s>>>(n, G, vis, valid, gcnt, core, dist16, B,
-                                                          locid, qloc, bytes);
+  ms_scatter<<<ms_blocks((u64)G * 64, MS_GRID), 256, 0, s>>>(n, G, vis, valid, gcnt, cbase, core, dist16,
+                                                          B, locid, ms_cols(valid), qloc, bytes);
   return hipGetLastError();
 }
 // Local degrees, then the hubs' unit offsets (nhubs may be 0).
@@ -849,10 +918,11 @@ extern "C" hipError_t scs_launch_ms_degree(const int32_t* adj, const MsUnit* uni
                                            u32* hubcnt, unsigned long long* bytes,
                                            hipStream_t s) {
   ms_degree<<<ms_blocks((u64)nunits * 64, MS_GRID), 256, 0, s>>>(adj, units, nunits, vis, valid,
-                                                                locid, B, hubcnt, bytes);
+                                                                locid, ms_cols(valid), B, hubcnt,
+                                                                bytes);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || nhubs == 0) return e;
-  ms_hubsum<<<ms_blocks((u64)nhubs * 64, MS_GRID), 256, 0, s>>>(hubs, nhubs, vis, valid, locid, B,
+  ms_hubsum<<<ms_blocks((u64)nhubs * 64, MS_GRID), 256, 0, s>>>(hubs, nhubs, vis, valid, locid, ms_cols(valid), B,
                                                              hubcnt, bytes);
   return hipGetLastError();
 }
@@ -870,11 +940,16 @@ extern "C" hipError_t scs_launch_ms_scan_loff(u32 nb, const MsBatch* B, u32* tot
   ms_loff_apply<<<blocks, 256, 0, s>>>(B, tot, valid, cmax, csum, bytes);
   return hipGetLastError();
 }
+// packed: the queries that scatter and degree took (valid may have lost some
+// since, for want of room; the rows keep their columns).
 extern "C" hipError_t scs_launch_ms_fill(const int32_t* adj, const MsUnit* units, u32 nunits,
-                                         const u64* vis, u64 valid, const u32* locid,
+                                         const u64* vis, u64 valid, u64 packed, const u32* locid,
                                          const MsBatch* B, const u32* hubcnt,
                                          unsigned long long* bytes, hipStream_t s) {
-  ms_fill<<<ms_blocks((u64)nunits * 64, MS_GRID), 256, 0, s>>>(adj, units, nunits, vis, valid,
-                                                              locid, B, hubcnt, bytes);
+  const u32 blocks = ms_blocks((u64)nunits * 64, MS_GRID);
+  if (__builtin_popcountll(valid) <= MS_FILL_FEW)
+    ms_fill<true><<<blocks, 256, 0, s>>>(adj, units, nunits, vis, valid, locid, ms_cols(packed), B, hubcnt, bytes);
+  else
+    ms_fill<false><<<blocks, 256, 0, s>>>(adj, units, nunits, vis, valid, locid, ms_cols(packed), B, hubcnt, bytes);
   return hipGetLastError();
 }
