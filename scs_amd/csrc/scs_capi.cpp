@@ -27,6 +27,9 @@ extern "C" {
 int scs_core_run(const i64* off, const int32_t* adj, u32 n, u32* core, u32* tmp,
                  hipStream_t s);
 u64 scs_core_words(u32 n);
+hipError_t scs_launch_csr_check(const i64* off, const int32_t* adj, u32 n, u64 nnz, u64* res,
+                                hipStream_t s);
+hipError_t scs_launch_csr_narrow(const i64* off, u32 n, u32* off32, u32* ident, hipStream_t s);
 hipError_t scs_launch_ms_init(u32 n, const u32* core, const MsBatch* B, u64* elig, u64* vis,
                               u64* fr, u64* nf, u64* xf, u32* flags, u32 nflags,
                               unsigned long long* bytes, hipStream_t s);
@@ -102,8 +105,7 @@ struct scs_graph {
 
 static int core_decompose(scs_graph* G) {
   const u32 n = G->hg.n;
-  hipStream_t s;
-  HIPCHK(hipStreamCreate(&s));
+  hipStream_t s = nullptr;
   u32* tmp;
   HIPCHK(hipMalloc(&tmp, sizeof(u32) * scs_core_words(n)));
   hipEvent_t e0, e1;
@@ -122,31 +124,65 @@ static int core_decompose(scs_graph* G) {
   HIPCHK(hipFree(tmp));
   HIPCHK(hipEventDestroy(e0));
   HIPCHK(hipEventDestroy(e1));
-  HIPCHK(hipStreamDestroy(s));
   return rc;
 }
 
-static int graph_upload(scs_graph* G) {
-  const u32 n = G->hg.n;
-  const u64 nnz = (u64)G->hg.off[n];
-  HIPCHK(hipMalloc(&G->d_off, sizeof(i64) * (n + 1)));
+// The CSR to the device, and what the host keeps of it.  check: the rows come
+// from a caller and are validated on the device before any other kernel reads
+// them; the host copies its own while that runs.
+static int graph_upload(scs_graph* G, const int64_t* off, const int32_t* adj, u32 n, u64 nnz,
+                        bool check) {
+  HIPCHK(hipMalloc(&G->d_off, sizeof(i64) * (n + 1ull)));
   HIPCHK(hipMalloc(&G->d_adj, sizeof(int32_t) * std::max<u64>(nnz, 1)));
-  HIPCHK(hipMalloc(&G->d_core, sizeof(u32) * std::max<u32>(n, 1)));
-  HIPCHK(hipMemcpy(G->d_off, G->hg.off.data(), sizeof(i64) * (n + 1), hipMemcpyHostToDevice));
-  if (nnz)
-    HIPCHK(hipMemcpy(G->d_adj, G->hg.adj.data(), sizeof(int32_t) * nnz, hipMemcpyHostToDevice));
-  G->hg.dmax = 0;
-  for (u32 v = 0; v < n; v++) G->hg.dmax = std::max<u32>(G->hg.dmax, (u32)(G->hg.off[v + 1] - G->hg.off[v]));
+  HIPCHK(hipMalloc(&G->d_core, sizeof(u32) * std::max<u64>(n, 32)));
+  HIPCHK(hipMemcpy(G->d_off, off, sizeof(i64) * (n + 1ull), hipMemcpyHostToDevice));
+  if (nnz) HIPCHK(hipMemcpy(G->d_adj, adj, sizeof(int32_t) * nnz, hipMemcpyHostToDevice));
+  u64* const res = (u64*)G->d_core;  // three words, before the core numbers are written
+  if (check && nnz) {
+    HIPCHK(hipMemset(res, 0, 3 * sizeof(u64)));
+    HIPCHK(scs_launch_csr_check(G->d_off, G->d_adj, n, nnz, res, nullptr));
+  }
   if (nnz <= 0xffffffffull) {
-    std::vector<u32> o32(n + 1), id(std::max<u32>(n, 1));
-    for (u32 v = 0; v <= n; v++) o32[v] = (u32)G->hg.off[v];
-    for (u32 v = 0; v < n; v++) id[v] = v;
-    HIPCHK(hipMalloc(&G->d_off32, sizeof(u32) * (n + 1)));
-    HIPCHK(hipMalloc(&G->d_ident, sizeof(u32) * id.size()));
-    HIPCHK(hipMemcpy(G->d_off32, o32.data(), sizeof(u32) * (n + 1), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(G->d_ident, id.data(), sizeof(u32) * id.size(), hipMemcpyHostToDevice));
+    HIPCHK(hipMalloc(&G->d_off32, sizeof(u32) * (n + 1ull)));
+    HIPCHK(hipMalloc(&G->d_ident, sizeof(u32) * std::max<u64>(n, 1)));
+    HIPCHK(scs_launch_csr_narrow(G->d_off, n, G->d_off32, G->d_ident, nullptr));
+  }
+  if (G->hg.off.empty()) {
+    G->hg.n = n;
+    G->hg.off.assign(off, off + n + 1);
+    G->hg.adj.assign(adj, adj + nnz);
+  }
+  G->hg.dmax = 0;
+  for (u32 v = 0; v < n; v++) G->hg.dmax = std::max<u32>(G->hg.dmax, (u32)(off[v + 1] - off[v]));
+  if (check && nnz) {
+    u64 got[3];
+    HIPCHK(hipMemcpy(got, res, sizeof(got), hipMemcpyDeviceToHost));
+    if ((u32)got[0] || got[1] != got[2]) return SCS_EINVAL;
   }
   return core_decompose(G);
+}
+
+// The same validation on the host, for a machine without a device: a bad CSR
+// is SCS_EINVAL there too.  Rows are visited in ascending v, so the entries
+// below w in row w must match, in order, the rows v < w that name w.
+static bool csr_valid_host(const int64_t* off, const int32_t* adj, u32 n, u64 nnz) {
+  for (u64 j = 0; j < nnz; j++)
+    if (adj[j] < 0 || (u32)adj[j] >= n) return false;
+  std::vector<i64> ptr(off, off + n);
+  for (u32 v = 0; v < n; v++) {
+    for (i64 j = off[v]; j < off[v + 1]; j++) {
+      const u32 w = (u32)adj[j];
+      if (w == v) return false;
+      if (j > off[v] && adj[j - 1] >= adj[j]) return false;
+      if (w > v) {
+        if (ptr[w] >= off[w + 1] || (u32)adj[ptr[w]] != v) return false;
+        ptr[w]++;
+      }
+    }
+    // every entry of row v below v must have been matched by now
+    if (ptr[v] < off[v + 1] && (u32)adj[ptr[v]] < v) return false;
+  }
+  return true;
 }
 
 extern "C" int scs_graph_create(const int64_t* off, const int32_t* adj, uint32_t n, uint64_t nnz,
@@ -156,33 +192,11 @@ extern "C" int scs_graph_create(const int64_t* off, const int32_t* adj, uint32_t
   if (off[0] != 0 || (u64)off[n] != nnz) return SCS_EINVAL;
   for (u32 v = 0; v < n; v++)
     if (off[v + 1] < off[v]) return SCS_EINVAL;
-  for (u64 j = 0; j < nnz; j++)
-    if (adj[j] < 0 || (u32)adj[j] >= n) return SCS_EINVAL;
-  // The search kernels need a simple undirected graph: every row strictly
-  // ascending (sorted, no duplicates), no self-loops, and w in row v exactly
-  // when v is in row w.  Rows are visited in ascending v, so the entries
-  // below w in row w must match, in order, the rows v < w that name w.
-  {
-    std::vector<i64> ptr(off, off + n);
-    for (u32 v = 0; v < n; v++) {
-      for (i64 j = off[v]; j < off[v + 1]; j++) {
-        const u32 w = (u32)adj[j];
-        if (w == v) return SCS_EINVAL;
-        if (j > off[v] && adj[j - 1] >= adj[j]) return SCS_EINVAL;
-        if (w > v) {
-          if (ptr[w] >= off[w + 1] || (u32)adj[ptr[w]] != v) return SCS_EINVAL;
-          ptr[w]++;
-        }
-      }
-      // every entry of row v below v must have been matched by now
-      if (ptr[v] < off[v + 1] && (u32)adj[ptr[v]] < v) return SCS_EINVAL;
-    }
-  }
+  int devices = 0;
+  if (hipGetDeviceCount(&devices) != hipSuccess || devices == 0)
+    return csr_valid_host(off, adj, n, nnz) ? SCS_EHIP : SCS_EINVAL;
   scs_graph* G = new scs_graph;
-  G->hg.n = n;
-  G->hg.off.assign(off, off + n + 1);
-  G->hg.adj.assign(adj, adj + nnz);
-  int rc = graph_upload(G);
+  int rc = graph_upload(G, off, adj, n, nnz, true);
   if (rc) {
     scs_graph_destroy(G);
     return rc;
@@ -238,7 +252,7 @@ extern "C" int scs_graph_load(const char* path, scs_graph** out) {
     G->hg.adj[i] = (int32_t)(keys[i] & 0xffffffffu);
   }
   for (u64 i = 0; i < n; i++) G->hg.off[i + 1] += G->hg.off[i];
-  int rc = graph_upload(G);
+  int rc = graph_upload(G, G->hg.off.data(), G->hg.adj.data(), (u32)n, keys.size(), false);
   if (rc) {
     scs_graph_destroy(G);
     return rc;

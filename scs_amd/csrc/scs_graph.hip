@@ -1,10 +1,95 @@
-// Graph-level kernels for gfx950: core decomposition, once per graph,
-// replacing the reference's host-side linear-heap peeling
-// (src/Graph.h:82-109).  Per-query preprocessing is batched in
+// Graph-level kernels for gfx950, once per graph: validation of a caller's CSR
+// and core decomposition, replacing the reference's host-side linear-heap
+// peeling (src/Graph.h:82-109).  Per-query preprocessing is batched in
 // scs_prep.hip.
 #include "scs_internal.h"
 
 #include <mutex>
+
+// ---------------------------------------------------------------------------
+// Validation of a caller's CSR (offsets checked by the host: they ascend from
+// 0 to nnz) and the 32-bit forms the search reads.  The search kernels need a
+// simple undirected graph: every row strictly ascending, ids inside [0, n), no
+// self-loops, and w in row v exactly when v is in row w.  A lane takes an
+// entry, finds its row by search over the offsets and, when w > v, looks v up
+// in row w; as many entries below the diagonal as above it leave none of those
+// unmatched.  Bound: the searches' dependent loads.  3M entries take 266 us,
+// 1,046 with a 16-lane segment per row (the longest row's), 4,000 on the host.
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(256) csr_check(const i64* __restrict__ off,
+                                                 const int32_t* __restrict__ adj, u32 n, u64 nnz,
+                                                 u32* __restrict__ bad,
+                                                 unsigned long long* __restrict__ above,
+                                                 unsigned long long* __restrict__ below) {
+  u64 up = 0, dn = 0;
+  bool wrong = false;
+  for (u64 j = (u64)blockIdx.x * blockDim.x + threadIdx.x; j < nnz;
+       j += (u64)gridDim.x * blockDim.x) {
+    u32 lo = 0, hi = n - 1;  // the last row whose offset is at most j
+    while (lo < hi) {
+      const u32 mid = lo + (hi - lo + 1) / 2;
+      if ((u64)off[mid] <= j)
+        lo = mid;
+      else
+        hi = mid - 1;
+    }
+    const u32 v = lo;
+    const int32_t w = adj[j];
+    if (w < 0 || (u32)w >= n || (u32)w == v || (j > (u64)off[v] && adj[j - 1] >= w)) {
+      wrong = true;
+      continue;
+    }
+    if ((u32)w < v) {
+      dn++;
+      continue;
+    }
+    up++;
+    i64 a = off[w], b = off[w + 1];  // first entry >= v
+    const i64 end = b;
+    while (a < b) {
+      const i64 mid = (a + b) >> 1;
+      if ((i64)adj[mid] < (i64)v)
+        a = mid + 1;
+      else
+        b = mid;
+    }
+    if (a == end || (i64)adj[a] != (i64)v) wrong = true;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    up += __shfl_xor(up, o);
+    dn += __shfl_xor(dn, o);
+  }
+  const bool any = __ballot(wrong) != 0;
+  if ((threadIdx.x & 63) == 0) {
+    if (any) atomicOr(bad, 1u);
+    if (up) atomicAdd(above, (unsigned long long)up);
+    if (dn) atomicAdd(below, (unsigned long long)dn);
+  }
+}
+__global__ void csr_narrow(const i64* __restrict__ off, u32 n, u32* __restrict__ off32,
+                           u32* __restrict__ ident) {
+  for (u64 v = (u64)blockIdx.x * blockDim.x + threadIdx.x; v <= n;
+       v += (u64)gridDim.x * blockDim.x) {
+    off32[v] = (u32)off[v];
+    if (v < n) ident[v] = (u32)v;
+  }
+}
+static u32 csr_blocks(u64 threads, u32 cap) {
+  const u64 b = (threads + 255) / 256;
+  return (u32)(b < 1 ? 1 : (b < cap ? b : cap));
+}
+// res: three u64 words, zeroed (bad, above, below).
+extern "C" hipError_t scs_launch_csr_check(const i64* off, const int32_t* adj, u32 n, u64 nnz,
+                                           u64* res, hipStream_t s) {
+  csr_check<<<csr_blocks(nnz, 2048), 256, 0, s>>>(
+      off, adj, n, nnz, (u32*)res, (unsigned long long*)(res + 1), (unsigned long long*)(res + 2));
+  return hipGetLastError();
+}
+extern "C" hipError_t scs_launch_csr_narrow(const i64* off, u32 n, u32* off32, u32* ident,
+                                            hipStream_t s) {
+  csr_narrow<<<csr_blocks((u64)n + 1, 2048), 256, 0, s>>>(off, n, off32, ident);
+  return hipGetLastError();
+}
 
 // ---------------------------------------------------------------------------
 // Core decomposition: level-synchronous peeling in one persistent kernel.
@@ -22,7 +107,7 @@
 // and its longest cascade (queue, offsets, neighbours, degree atomics: 4 us a
 // step); the innermost core, thousands of hubs that leave together, is bound
 // by atomics on the same degrees (2 ms).  Chung-Lu graphs, 88K / 1.5M / 8M
-// edges (16 / 76 / 206 levels): 0.47 / 1.9 / 7.0 ms, 3.0 / 17.0 / 40.7 ms
+// edges (16 / 76 / 206 levels): 0.43 / 1.9 / 6.7 ms, 3.0 / 17.0 / 40.7 ms
 // before, with a launch and a host round trip per cascade step.  Blocks of
 // 256 and 1,024 threads are 2-12 % slower on these three, 2,048 vertices per
 // block and more 1.5 times slower on the first.
@@ -75,10 +160,11 @@ __global__ void core_init(const i64* __restrict__ off, u32 n, u32* __restrict__ 
                           CoreCtl* __restrict__ ctl) {
   for (u32 v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
     deg[core_pos(v, mask)] = (u32)(off[v + 1] - off[v]);
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    CoreCtl c{};
-    c.minrest = 0xffffffffu;
-    *ctl = c;  // one thread: a few hundred words, once per run
+  if (blockIdx.x == 0) {
+    u32* w = (u32*)ctl;
+    for (u32 i = threadIdx.x; i < sizeof(CoreCtl) / 4; i += blockDim.x) w[i] = 0;
+    __syncthreads();
+    if (threadIdx.x == 0) ctl->minrest = 0xffffffffu;
   }
 }
 

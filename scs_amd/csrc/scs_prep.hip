@@ -301,20 +301,21 @@ __global__ void __launch_bounds__(256) ms_level(const int32_t* __restrict__ adj,
   ms_count_bytes(bytes, nbytes);
 }
 
-// Kept counts.  A wave takes MS_CHUNK groups of 64 vertices, lane b counting
+// Kept counts.  A wave takes a chunk of `ch` groups of 64 vertices, lane b counting
 // for query b: gcnt[g * 64 + b] = query b's kept vertices in the chunk's groups
 // before g, cbase[c * 64 + b] = those in chunk c.  vis takes in the last
-// level's finds (lf; bits already there when the search ended earlier).
-#define MS_CHUNK 32
-__global__ void __launch_bounds__(256) ms_count(u32 n, u32 G, u64* __restrict__ vis,
+// level's finds (lf; bits already there when the search ended earlier).  At
+// most 256 chunks: enough waves for the count, and few rows for the one wave
+// that scans them.
+__global__ void __launch_bounds__(256) ms_count(u32 n, u32 G, u32 ch, u64* __restrict__ vis,
                                                 const u64* __restrict__ lf, u64 valid,
                                                 u32* __restrict__ gcnt, u32* __restrict__ cbase,
                                                 unsigned long long* bytes) {
   const u32 lane = threadIdx.x & 63;
   const u32 c = ms_wave_id();
-  const u32 g0 = c * MS_CHUNK;
+  const u32 g0 = c * ch;
   if (g0 >= G) return;
-  const u32 g1 = min(G, g0 + MS_CHUNK);
+  const u32 g1 = min(G, g0 + ch);
   u64 nbytes = 0;
   u32 run = 0;
   for (u32 g = g0; g < g1; g += 8) {
@@ -376,7 +377,8 @@ struct MsCols {
 };
 
 // Local ids, and per kept vertex: orig id, distance, core number.
-__global__ void __launch_bounds__(256) ms_scatter(u32 n, u32 G, const u64* __restrict__ vis,
+__global__ void __launch_bounds__(256) ms_scatter(u32 n, u32 G, u32 ch,
+                                                  const u64* __restrict__ vis,
                                                   u64 valid, const u32* __restrict__ gcnt,
                                                   const u32* __restrict__ cbase,
                                                   const u32* __restrict__ core,
@@ -398,7 +400,7 @@ __global__ void __launch_bounds__(256) ms_scatter(u32 n, u32 G, const u64* __res
     const u64 v = (u64)g * 64 + lane;
     const u64 m = v < n ? vis[v] & valid : 0;
     // lane b: query b's first id in the group
-    const u32 gb = gcnt[(u64)g * 64 + lane] + cbase[(u64)(g / MS_CHUNK) * 64 + lane];
+    const u32 gb = gcnt[(u64)g * 64 + lane] + cbase[(u64)(g / ch) * 64 + lane];
     u32 cv = 0;
     if (m) {
       cv = core[v];
@@ -883,19 +885,20 @@ extern "C" hipError_t scs_launch_ms_level(const int32_t* adj, const MsUnit* unit
       flag_cur, bytes);
   return hipGetLastError();
 }
+static u32 ms_chunk(u32 G) { return G ? (G + 255) / 256 : 1; }
 // Kept counts and their bases: gcnt holds G * 64 words, cbase one row of 64
-// per MS_CHUNK groups.
+// per chunk.
 extern "C" hipError_t scs_launch_ms_count(u32 n, u32 G, u64* vis, const u64* lf, u64 valid,
                                           u32* gcnt, u32* cbase, u32* tot,
                                           unsigned long long* bytes, hipStream_t s) {
-  const u32 C = (G + MS_CHUNK - 1) / MS_CHUNK;
-  if (C) ms_count<<<(C + 3) / 4, 256, 0, s>>>(n, G, vis, lf, valid, gcnt, cbase, bytes);
+  const u32 ch = ms_chunk(G), C = (G + ch - 1) / ch;
+  if (C) ms_count<<<(C + 3) / 4, 256, 0, s>>>(n, G, ch, vis, lf, valid, gcnt, cbase, bytes);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   ms_bscan<<<1, 64, 0, s>>>(C, cbase, tot, bytes);
   return hipGetLastError();
 }
-extern "C" u64 scs_ms_count_rows(u32 G) { return (G + MS_CHUNK - 1) / MS_CHUNK; }
+extern "C" u64 scs_ms_count_rows(u32 G) { return G ? (G + ms_chunk(G) - 1) / ms_chunk(G) : 1; }
 extern "C" hipError_t scs_launch_ms_gdist(u32 n, u32 G, const u64* vis, u64 gmask,
                                           const u16* dist16, const MsBatch* B,
                                           unsigned long long* bytes, hipStream_t s) {
@@ -907,7 +910,8 @@ extern "C" hipError_t scs_launch_ms_scatter(u32 n, u32 G, const u64* vis, u64 va
                                             const u16* dist16,
                                             const MsBatch* B, u32* locid, u32* qloc,
                                             unsigned long long* bytes, hipStream_t s) {
-  ms_scatter<<<ms_blocks((u64)G * 64, MS_GRID), 256, 0, s>>>(n, G, vis, valid, gcnt, cbase, core, dist16,
+  ms_scatter<<<ms_blocks((u64)G * 64, MS_GRID), 256, 0, s>>>(n, G, ms_chunk(G), vis, valid, gcnt, cbase,
+                                                          core, dist16,
                                                           B, locid, ms_cols(valid), qloc, bytes);
   return hipGetLastError();
 }
