@@ -1930,6 +1930,96 @@ __device__ __forceinline__ void rebuild(W& w, const u32* task) {
   wsync();
 }
 
+// The next level's root from the one this wave has just searched (form 2 both,
+// the state's trail still holds the old root's closure).  A lower bound only
+// adds vertices: R_old = {core > root_kl, within ubD(root_kl)} is part of the
+// new R, so the old root's counts stand once its trail is undone, and only the
+// adjacency of the vertices that join is read.  root_kl is the bound R was
+// built for; returns the new one.
+//
+// A rebuild reads the adjacency of all of R at every level (3.4 ms of a wave
+// on a 50,000-vertex, 750,000-edge graph, 30 levels and more per query); over
+// a query's levels this reads each list once.  The batch of 64 such queries
+// (16 nodes each) takes 130 ms, 177 with rebuilt roots.
+__device__ __forceinline__ u32 grow_root(W& w, u32 kl) {
+  undo_to<4>(w, 0);
+  const u32 K = w.K, ub = ubd_node(kl, w.h), q0 = w.clist[0], nR = w.nR;
+  const u32 nw = (K + 31) / 32;
+  u32 cnt = 0;
+  for (u32 v0 = 0; v0 < K; v0 += 512) {
+    u32 cr[8], ds[8];
+    u8 st[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const u32 v = min(v0 + 64u * k + LANE, K - 1);
+      cr[k] = w.core[v];
+      ds[k] = w.dist[v];
+      st[k] = w.bm ? (u8)(xbit(w, v) ? ST_X : ST_R) : w.vs[v].st;
+    }
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const u32 c0 = v0 + 64u * k;
+      if (c0 >= K) break;
+      const u32 v = c0 + LANE;
+      const bool join = v < K && st[k] == ST_X && cr[k] > kl && ds[k] <= ub;
+      const u64 m = __ballot(join);
+      if (!m) continue;
+      if (join) {
+        const u32 p = cnt + __popcll(m & lanes_below());
+        w.vs[v].st = ST_R;
+        w.work[p] = v;
+        w.rlist[nR + p] = v;
+        w.pos[v] = nR + p;
+        if (!w.bm) w.nmark[v] = 1;
+      }
+      if (w.bm) {
+        // tb = the vertices that join
+        const u32 i = (c0 >> 5) + LANE;
+        const u32 mw = LANE ? (u32)(m >> 32) : (u32)m;
+        if (LANE < 2 && i < nw) {
+          w.xb[i] &= ~mw;
+          w.tb[i] = mw;
+        }
+      }
+      cnt += __popcll(m);
+    }
+  }
+  wsync();
+  const u32* jn = w.work;
+  const bool bm = w.bm;
+  enum : u32 { NX, NC, NJOIN, NOLD };  // of a neighbour: removed, q, joining, already in R
+  scan_adj<u64, true>(
+      w, cnt, [&](u32 i) { return jn[i]; },
+      [&](u32 x, bool) -> u32 {
+        if (x == q0) return NC;
+        if (bm) return xbit(w, x) ? NX : (tbit(w, x) ? NJOIN : NOLD);
+        return w.vs[x].st == ST_X ? NX : (w.nmark[x] ? NJOIN : NOLD);
+      },
+      [&](u32 x, u32 t) -> u64 {
+        if (t == NX) return 0;
+        if (t != NJOIN) atomicAdd(&w.vs[x].dR, 1u);
+        return t == NC ? 1ull << 32 : 1ull;
+      },
+      [&](u32, u32 v, u64 cr) {
+        const u32 c = (u32)(cr >> 32);
+        w.vs[v].dC = (u16)c;
+        w.vs[v].dR = (u32)cr;
+        atomicAdd(&w.L->hist[min(c, w.h + 1)], 1u);
+      });
+  wsync();
+  if (bm) {
+    for (u32 i = LANE; i < nw; i += 64) w.tb[i] = 0;
+  } else {
+    for (u32 i = LANE; i < cnt; i += 64) w.nmark[w.work[i]] = 0;
+  }
+  w.nR = nR + cnt;
+  w.ntrail = 0;
+  w.nframes = 0;
+  w.nsav = 0;
+  wsync();
+  return kl;
+}
+
 // Serialises the Z child of frame fi (the unexplored "exclude u*" branch)
 // into dst (dst[3] = form set by the caller: 1 = list R, 0 = list X);
 // returns the payload length in words.
@@ -1987,7 +2077,8 @@ __device__ __forceinline__ u32 serialize_z(W& w, u32 fi, u32* dst, u32 qslot) {
   return 4 + f.csize + base;
 }
 
-__device__ __forceinline__ void save_state(W& w, u32 active, u32 qslot, u32 from, u32 kl_seen) {
+__device__ __forceinline__ void save_state(W& w, u32 active, u32 qslot, u32 from, u32 kl_seen,
+                                           u32 root_kl) {
   if (active)
     for (u32 i = LANE; i < SCS_HCAP + 4; i += 64) w.ghist[i] = w.L->hist[i];
   if (LANE == 0) {
@@ -2002,6 +2093,7 @@ __device__ __forceinline__ void save_state(W& w, u32 active, u32 qslot, u32 from
     H->kl_seen = kl_seen;
     H->pend_nodes = 0;
     H->nsav = w.nsav;
+    H->root_kl = root_kl;
   }
   wsync();
 }
@@ -2081,6 +2173,9 @@ __global__ void __launch_bounds__(64, 2) __attribute__((flatten)) scs_epoch(Engi
   WaveHdr* H = w.hdr;
   u32 active = H->active, qslot = H->qslot;
   u32 from = H->from, kl_seen = H->kl_seen, pend = 0;
+  // the bound of the level root this wave's state was built for (INV: the task
+  // is not a level's root)
+  u32 root_kl = H->root_kl;
   if (active) {
     bind_query(w, &A.slots[qslot]);
     w.nframes = H->nframes;
@@ -2138,6 +2233,7 @@ __global__ void __launch_bounds__(64, 2) __attribute__((flatten)) scs_epoch(Engi
         continue;
       }
       ph_switch(&L, tp, ph, PH_REBUILD);
+      root_kl = task[3] == 2 ? cur_kl(w) : INV;
       rebuild(w, task);  // ends in a barrier: the payload has been read
       if (LANE == 0) {
         astore64(&A.pool.seq[pos % A.pool.nslots], pos + A.pool.nslots);
@@ -2239,7 +2335,13 @@ __global__ void __launch_bounds__(64, 2) __attribute__((flatten)) scs_epoch(Engi
         if (finish_task(w, A, qslot)) {
           // the query's next level: its root, searched by this wave
           ph_switch(&L, tp, ph, PH_REBUILD);
-          rebuild(w, L.root);
+          const u32 kl = cur_kl(w);
+          if (kl <= root_kl && root_kl != INV) {
+            root_kl = grow_root(w, kl);
+          } else {
+            root_kl = kl;
+            rebuild(w, L.root);
+          }
           active = 1;
           from = 0;
           kl_seen = INV;
@@ -2305,9 +2407,9 @@ __global__ void __launch_bounds__(64, 2) __attribute__((flatten)) scs_epoch(Engi
     atomicAdd((unsigned long long*)&A.glob->tph[LANE], (unsigned long long)L.tph[LANE]);
   if (active) {
     flush_counters(w, A, pend);
-    save_state(w, 1, qslot, from, kl_seen);
+    save_state(w, 1, qslot, from, kl_seen, root_kl);
   } else {
-    save_state(w, 0, 0, 0, INV);
+    save_state(w, 0, 0, 0, INV, INV);
   }
 }
 

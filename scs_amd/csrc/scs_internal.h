@@ -96,7 +96,8 @@ struct WaveHdr {
   u32 pend_nodes;// nodes not yet added to the query counter
   u32 pend_edges;// adjacency entries not yet added to the global counter
   u32 nsav;      // words on the recount save stack
-  u32 pad[4];
+  u32 root_kl;   // bound of the level root the state was built for
+  u32 pad[3];
 };
 
 // Search state of one vertex, packed so that the fields a rule or counter
