@@ -278,8 +278,8 @@ __device__ __forceinline__ void build_bitmaps(W& w) {
 // graph takes 3.4 ms, 16 ms with one 64-entry chunk of one vertex at a time.
 // With the loops over R and the trail taking 4 to 8 vertices per lane at once
 // and the shared words polled without fences, a batch of 64 queries of that
-// graph (16 nodes each) takes 177 ms instead of 1,236 ms, and a 64-query
-// batch of proofs on 20,000 vertices 44 ms instead of 243 ms.
+// graph (16 nodes each) went from 1,236 to 177 ms, and a 64-query
+// batch of proofs on 20,000 vertices from 243 to 44 ms.
 // ---------------------------------------------------------------------------
 #define SEQ_DEG 32u
 #define HUB_DEG 512u
@@ -938,6 +938,16 @@ __device__ __forceinline__ void try_push(W& w, u32 x, u64 wd, u32 ds, u32 Cs, u3
 // (|C| grew), or everything when kl changed.  Each round removes all
 // queued vertices as one batch and queues the neighbours it pushes below
 // the rule-1 threshold.  Returns true if anything was removed.
+//
+// Bound by the gathers of state words and distances, one cache line per entry.
+// When the removed vertices' lists hold more entries than R has vertices, all
+// of R is looked at instead: it finds the same vertices, each looked at once.
+// And when R is at least half of the kept set, that look takes the state
+// records in id order, not R's order, which removals have shuffled: whole
+// lines instead of one per vertex (50,000 vertices: 0.1 ms instead of 1 ms).
+// Eight batches of 64 queries (16 nodes each, 50,000 vertices, 750,000 edges):
+// 738 ms, 796 with the lists alone left out, 1,058 before; either line could
+// lie a factor of two to each side (798 to 808, 738 to 740 ms).
 __device__ __forceinline__ bool r12(W& w, u32 from, bool full, u32 kl, u64& tp, u32& ph) {
   Lds* L = w.L;
   const u32 Cs = w.nC;
@@ -954,6 +964,34 @@ __device__ __forceinline__ bool r12(W& w, u32 from, bool full, u32 kl, u64& tp, 
       if (wsum(c)) full = true;
     }
   }
+  u32 nrm = 0;
+  if (!full) {
+    // vertices removed since `from` (trail entries without the move or
+    // batch-marker flags), compacted into work2
+    u64 deg = 0;
+    for (u32 t0 = from; t0 < w.ntrail && !full; t0 += 256) {
+      u32 e[4], b[4], n[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const u32 t = t0 + 64u * k + LANE;
+        e[k] = w.trail[min(t, w.ntrail - 1)];
+        if (t >= w.ntrail) e[k] = TR_MARK;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const bool plain = !(e[k] & (TR_MOVE | TR_MARK));
+        b[k] = plain ? w.off[e[k]] : 0u;
+        n[k] = plain ? w.off[e[k] + 1] : 0u;
+        const u64 bm = __ballot(plain);
+        if (plain) w.work2[nrm + __popcll(bm & lanes_below())] = e[k];
+        nrm += __popcll(bm);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++) deg += n[k] - b[k];
+      full = wsum64(deg) > w.nR;
+    }
+    wsync();
+  }
   if (full) {
     if (LANE == 0) {
       atomicAdd((unsigned long long*)&w.gl->full_scans, 1ull);
@@ -962,12 +1000,16 @@ __device__ __forceinline__ bool r12(W& w, u32 from, bool full, u32 kl, u64& tp, 
     // eight R vertices per lane per step: the list loads, then their
     // state words and distances, are in flight together (indices past the
     // list's end read its last entry and are ignored)
-    const u32 nR = w.nR;
     const bool r2 = w.flags & QF_RED2;
+    const bool lin = 2ull * w.nR >= w.K;
+    const u32 nR = lin ? w.K : w.nR;
     for (u32 i0 = 0; i0 < nR; i0 += 512) {
       u32 x[8];
 #pragma unroll
-      for (int k = 0; k < 8; k++) x[k] = w.rlist[min(i0 + LANE + 64u * k, nR - 1)];
+      for (int k = 0; k < 8; k++) {
+        x[k] = min(i0 + LANE + 64u * k, nR - 1);
+        if (!lin) x[k] = w.rlist[x[k]];
+      }
       u64 wd[8];
       u32 ds[8];
 #pragma unroll
@@ -979,27 +1021,6 @@ __device__ __forceinline__ bool r12(W& w, u32 from, bool full, u32 kl, u64& tp, 
         if (i0 + LANE + 64u * k < nR) try_push(w, x[k], wd[k], ds[k], Cs, ubD, kl, w.work, &L->cnt);
     }
   } else {
-    // vertices removed since `from` (trail entries without the move or
-    // batch-marker flags), compacted into work2, then their neighbours
-    // checked with the load-balanced scan
-    u32 nrm = 0;
-    for (u32 t0 = from; t0 < w.ntrail; t0 += 256) {
-      u32 e[4];
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const u32 t = t0 + 64u * k + LANE;
-        e[k] = w.trail[min(t, w.ntrail - 1)];
-        if (t >= w.ntrail) e[k] = TR_MARK;
-      }
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const bool plain = !(e[k] & (TR_MOVE | TR_MARK));
-        const u64 bm = __ballot(plain);
-        if (plain) w.work2[nrm + __popcll(bm & lanes_below())] = e[k];
-        nrm += __popcll(bm);
-      }
-    }
-    wsync();
     if (nrm) {
       const u32* rm = w.work2;
       struct WD {
