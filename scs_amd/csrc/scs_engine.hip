@@ -44,6 +44,10 @@ __device__ __forceinline__ u32 wmin(u32 x) {
   for (int o = 32; o > 0; o >>= 1) x = min(x, (u32)__shfl_xor((int)x, o));
   return x;
 }
+__device__ __forceinline__ u32 wmax(u32 x) {
+  for (int o = 32; o > 0; o >>= 1) x = max(x, (u32)__shfl_xor(x, o));
+  return x;
+}
 __device__ __forceinline__ u32 wsum(u32 x) {
   for (int o = 32; o > 0; o >>= 1) x += (u32)__shfl_xor((int)x, o);
   return x;
@@ -262,7 +266,9 @@ __device__ __forceinline__ void build_bitmaps(W& w) {
 // or an atomic when `in`; entries that are not `in` pad a step and are
 // ignored), edge(x, t) turns what came back into a contribution (AccT), and
 // done(i, v, total) runs once per vertex with the sum of its contributions,
-// on one lane (SUM = false: no sums, done is not called).
+// on one lane (SUM = false: no sums, done is not called).  scan_adj2 has a
+// look(x, in) before load, whose results decide what load(x, look) does and
+// which are all read before the first load.
 //
 // One wave per SIMD runs, so nothing but the wave's own independent loads
 // hides a memory round trip: every path keeps several entries per lane in
@@ -272,7 +278,12 @@ __device__ __forceinline__ void build_bitmaps(W& w) {
 // as one concatenated list, 256 entries a step, the owner of an entry found
 // by binary search over the lanes' exclusive degree sums: a list below
 // SEQ_DEG is read in at most eight steps of its lane, and above HUB_DEG the
-// search would cost more than the loads it balances.
+// search would cost more than the loads it balances.  Where 64 lists are
+// together at least half of 64 times their longest, all up to HUB_DEG are
+// taken one per lane: on a power-law graph, whose ids follow the degrees, a
+// search of 16 nodes takes 15.9 instead of 20.7 ms on average (a quarter:
+// 16.1, three quarters: 17.2).  A fixed line at 128 entries gives 17.7 there
+// and costs 4% on graphs whose ids do not.
 //
 // A level root's neighbour count on a 50,000-vertex, 750,000-edge power-law
 // graph takes 3.4 ms, 16 ms with one 64-entry chunk of one vertex at a time.
@@ -291,11 +302,12 @@ __device__ __forceinline__ u32 wsum_t<u32>(u32 x) { return wsum(x); }
 template <>
 __device__ __forceinline__ u64 wsum_t<u64>(u64 x) { return wsum64(x); }
 
-template <typename AccT, bool SUM, typename VertexF, typename LoadF, typename EdgeF,
-          typename DoneF>
-__device__ __forceinline__ void scan_adj(W& w, u32 m, VertexF vertex, LoadF load, EdgeF edge,
-                                         DoneF done) {
-  using T = decltype(load(0u, true));
+template <typename AccT, bool SUM, typename VertexF, typename LookF, typename LoadF,
+          typename EdgeF, typename DoneF>
+__device__ __forceinline__ void scan_adj2(W& w, u32 m, VertexF vertex, LookF look, LoadF load,
+                                          EdgeF edge, DoneF done) {
+  using P = decltype(look(0u, true));
+  using T = decltype(load(0u, P()));
   u32 ed = 0;
   u32 vn = 0, bn = 0, en = 0;  // the next 64 vertices
   if (LANE < m) {
@@ -313,8 +325,15 @@ __device__ __forceinline__ void scan_adj(W& w, u32 m, VertexF vertex, LoadF load
     }
     const bool on = i < m;
     const u32 deg = on ? e - b : 0u;
-    const bool mid = deg > SEQ_DEG && deg <= HUB_DEG;
-    if (on && deg <= SEQ_DEG) {
+    // lists of much the same length are read best one per lane, whatever the
+    // length: no search, and no lane waits long for another
+    u32 seq = SEQ_DEG;
+    if (__ballot(deg > SEQ_DEG && deg <= HUB_DEG)) {
+      const u32 dl = deg <= HUB_DEG ? deg : 0u;
+      if (2 * wsum(dl) >= 64u * wmax(dl)) seq = HUB_DEG;
+    }
+    const bool mid = deg > seq && deg <= HUB_DEG;
+    if (on && deg <= seq) {
       AccT acc = 0;
       if (deg) {
         u32 x[4];
@@ -322,11 +341,14 @@ __device__ __forceinline__ void scan_adj(W& w, u32 m, VertexF vertex, LoadF load
         for (int k = 0; k < 4; k++) x[k] = w.adj[min(b + k, e - 1)];
         for (u32 j = b; j < e; j += 4) {
           u32 xn[4];
+          P p[4];
           T t[4];
 #pragma unroll
           for (int k = 0; k < 4; k++) xn[k] = w.adj[min(j + 4 + k, e - 1)];
 #pragma unroll
-          for (int k = 0; k < 4; k++) t[k] = load(x[k], j + k < e);
+          for (int k = 0; k < 4; k++) p[k] = look(x[k], j + k < e);
+#pragma unroll
+          for (int k = 0; k < 4; k++) t[k] = load(x[k], p[k]);
 #pragma unroll
           for (int k = 0; k < 4; k++)
             if (j + k < e) acc += edge(x[k], t[k]);
@@ -368,10 +390,13 @@ __device__ __forceinline__ void scan_adj(W& w, u32 m, VertexF vertex, LoadF load
       fetch(0, x, own);
       for (u32 k0 = 0; k0 < tot; k0 += 64 * U) {
         u32 xn[U], on2[U];
+        P p[U];
         T t[U];
         if (k0 + 64 * U < tot) fetch(k0 + 64 * U, xn, on2);
 #pragma unroll
-        for (int k = 0; k < U; k++) t[k] = load(x[k], k0 + 64 * k + LANE < tot);
+        for (int k = 0; k < U; k++) p[k] = look(x[k], k0 + 64 * k + LANE < tot);
+#pragma unroll
+          for (int k = 0; k < U; k++) t[k] = load(x[k], p[k]);
 #pragma unroll
         for (int k = 0; k < U; k++)
           if (k0 + 64 * k + LANE < tot) {
@@ -403,11 +428,14 @@ __device__ __forceinline__ void scan_adj(W& w, u32 m, VertexF vertex, LoadF load
       for (int k = 0; k < U; k++) x[k] = w.adj[min(bb + LANE + 64u * k, be - 1)];
       for (u32 j = bb + LANE; j - LANE < be; j += 64 * U) {
         u32 xn[U];
+        P p[U];
         T t[U];
 #pragma unroll
         for (int k = 0; k < U; k++) xn[k] = w.adj[min(j + 64u * (U + k), be - 1)];
 #pragma unroll
-        for (int k = 0; k < U; k++) t[k] = load(x[k], j + 64u * k < be);
+        for (int k = 0; k < U; k++) p[k] = look(x[k], j + 64u * k < be);
+#pragma unroll
+          for (int k = 0; k < U; k++) t[k] = load(x[k], p[k]);
 #pragma unroll
         for (int k = 0; k < U; k++)
           if (j + 64u * k < be) acc += edge(x[k], t[k]);
@@ -422,6 +450,13 @@ __device__ __forceinline__ void scan_adj(W& w, u32 m, VertexF vertex, LoadF load
     }
   }
   w.edges += wsum(ed);
+}
+
+template <typename AccT, bool SUM, typename VertexF, typename LoadF, typename EdgeF,
+          typename DoneF>
+__device__ __forceinline__ void scan_adj(W& w, u32 m, VertexF vertex, LoadF load, EdgeF edge,
+                                         DoneF done) {
+  scan_adj2<AccT, SUM>(w, m, vertex, [](u32, bool in) { return in; }, load, edge, done);
 }
 
 // Adds delta to hist[d] for every lane with `on` (call on all lanes).  Most
@@ -554,76 +589,18 @@ __device__ __forceinline__ void dec_neighbour(W& w, u32 x, const Clo& c) {
   dec_check(w, x, old, c);
 }
 
-// Decrements dR of every live neighbour of list[0..m) (load-balanced like
-// scan_adj).  Four entries per lane per step, software-pipelined: the next
-// step's adjacency loads are issued before this step's decrements, so one
-// memory round trip covers both (the memory counter is in order).  Loads
-// past a list's end read its last entry (or entry 0 of an empty graph) and
-// are ignored.
-__device__ __forceinline__ void dec4(W& w, const u32 x[4], const bool in[4], const Clo& c) {
-  bool lv[4];
-  u64 od[4];
-#pragma unroll
-  for (int k = 0; k < 4; k++) lv[k] = in[k] && dec_live(w, x[k]);
-#pragma unroll
-  for (int k = 0; k < 4; k++)
-    od[k] = lv[k] ? atomicSub((unsigned long long*)&w.vs[x[k]], 1ull) : 0ull;
-#pragma unroll
-  for (int k = 0; k < 4; k++)
-    if (lv[k]) dec_check(w, x[k], od[k], c);
-}
+// Decrements dR of every live neighbour of list[0..m).
 __device__ __forceinline__ void dec_neighbours(W& w, const u32* list, u32 m, const Clo& c) {
-  u32 ed = 0;
-  for (u32 c0 = 0; c0 < m; c0 += 64) {
-    const u32 i = c0 + LANE;
-    u32 v = 0, b = 0, e = 0;
-    if (i < m) {
-      v = list[i];
-      b = w.off[v];
-      e = w.off[v + 1];
-    }
-    const bool big = i < m && (e - b) > SEQ_DEG;
-    if (i < m && !big && e > b) {
-      u32 x[4];
-#pragma unroll
-      for (int k = 0; k < 4; k++) x[k] = w.adj[min(b + k, e - 1)];
-      for (u32 j = b; j < e; j += 4) {
-        u32 xn[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) xn[k] = w.adj[min(j + 4 + k, e - 1)];
-        bool in[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) in[k] = j + k < e;
-        dec4(w, x, in, c);
-#pragma unroll
-        for (int k = 0; k < 4; k++) x[k] = xn[k];
-      }
-      ed += e - b;
-    }
-    u64 bm = __ballot(big);
-    while (bm) {
-      const int src = __ffsll((unsigned long long)bm) - 1;
-      bm &= bm - 1;
-      const u32 bb = __shfl(b, src), be = __shfl(e, src);
-      // the whole wave, 256 entries per step
-      u32 x[4];
-#pragma unroll
-      for (int k = 0; k < 4; k++) x[k] = w.adj[min(bb + LANE + 64 * k, be - 1)];
-      for (u32 j = bb; j < be; j += 256) {
-        u32 xn[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) xn[k] = w.adj[min(j + 256 + LANE + 64 * k, be - 1)];
-        bool in[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) in[k] = j + LANE + 64 * k < be;
-        dec4(w, x, in, c);
-#pragma unroll
-        for (int k = 0; k < 4; k++) x[k] = xn[k];
-      }
-      if (LANE == 0) ed += be - bb;
-    }
-  }
-  w.edges += wsum(ed);
+  scan_adj2<u32, false>(
+      w, m, [&](u32 i) { return list[i]; }, [&](u32 x, bool in) { return in && dec_live(w, x); },
+      [&](u32 x, bool live) {
+        return live ? atomicSub((unsigned long long*)&w.vs[x], 1ull) : (u64)ST_X << 48;
+      },
+      [&](u32 x, u64 old) {
+        dec_check(w, x, old, c);
+        return 0u;
+      },
+      [&](u32, u32, u32) {});
 }
 
 // Removes the m vertices of list (all currently R) as one trail batch.
