@@ -1938,7 +1938,8 @@ __device__ __forceinline__ void rebuild(W& w, const u32* task) {
 // A rebuild reads the adjacency of all of R at every level (3.4 ms of a wave
 // on a 50,000-vertex, 750,000-edge graph, 30 levels and more per query); over
 // a query's levels this reads each list once.  The batch of 64 such queries
-// (16 nodes each) takes 130 ms, 177 with rebuilt roots.
+// (16 nodes each) went from 177 to 130 ms with it; with the closure's choice
+// (r12) and the even lists (scan_adj) it takes 75 to 94 ms.
 __device__ __forceinline__ u32 grow_root(W& w, u32 kl) {
   undo_to<4>(w, 0);
   const u32 K = w.K, ub = ubd_node(kl, w.h), q0 = w.clist[0], nR = w.nR;
