@@ -279,11 +279,16 @@ __device__ __forceinline__ void build_bitmaps(W& w) {
 // by binary search over the lanes' exclusive degree sums: a list below
 // SEQ_DEG is read in at most eight steps of its lane, and above HUB_DEG the
 // search would cost more than the loads it balances.  Where 64 lists are
-// together at least half of 64 times their longest, all up to HUB_DEG are
-// taken one per lane: on a power-law graph, whose ids follow the degrees, a
-// search of 16 nodes takes 15.9 instead of 20.7 ms on average (a quarter:
-// 16.1, three quarters: 17.2).  A fixed line at 128 entries gives 17.7 there
-// and costs 4% on graphs whose ids do not.
+// together at least half of 64 times their longest, those up to EVEN_DEG are
+// taken one per lane.
+//
+// Where the lines lie: a search that fills the chip (100 queries on 4,000
+// vertices and 88,000 edges, 195,000 entries a node, most in the pair rule) runs 476,000 nodes
+// a second with 128 and 256; 387,000 to 403,000 with both at 512, 421,000 with
+// 512 and no even lists, 484,000 with 96 and 96, 453,000 with 96 and 512.
+// Eight batches of 64 queries on a 50,000-vertex power-law graph, whose ids
+// follow the degrees, take 615 ms with 128 and 256; 618 to 650 with 512 and
+// 512, 725 without even lists, 645 with 96 and 96, 603 with 96 and 512.
 //
 // A level root's neighbour count on a 50,000-vertex, 750,000-edge power-law
 // graph takes 3.4 ms, 16 ms with one 64-entry chunk of one vertex at a time.
@@ -293,7 +298,8 @@ __device__ __forceinline__ void build_bitmaps(W& w) {
 // batch of proofs on 20,000 vertices from 243 to 44 ms.
 // ---------------------------------------------------------------------------
 #define SEQ_DEG 32u
-#define HUB_DEG 512u
+#define HUB_DEG 128u
+#define EVEN_DEG 256u
 
 template <typename AccT>
 __device__ __forceinline__ AccT wsum_t(AccT x);
@@ -328,9 +334,9 @@ __device__ __forceinline__ void scan_adj2(W& w, u32 m, VertexF vertex, LookF loo
     // lists of much the same length are read best one per lane, whatever the
     // length: no search, and no lane waits long for another
     u32 seq = SEQ_DEG;
-    if (__ballot(deg > SEQ_DEG && deg <= HUB_DEG)) {
-      const u32 dl = deg <= HUB_DEG ? deg : 0u;
-      if (2 * wsum(dl) >= 64u * wmax(dl)) seq = HUB_DEG;
+    if (__ballot(deg > SEQ_DEG && deg <= EVEN_DEG)) {
+      const u32 dl = deg <= EVEN_DEG ? deg : 0u;
+      if (2 * wsum(dl) >= 64u * wmax(dl)) seq = EVEN_DEG;
     }
     const bool mid = deg > seq && deg <= HUB_DEG;
     if (on && deg <= seq) {
@@ -416,7 +422,7 @@ __device__ __forceinline__ void scan_adj2(W& w, u32 m, VertexF vertex, LookF loo
       }
       ed += dm;
     }
-    u64 hubs = __ballot(deg > HUB_DEG);
+    u64 hubs = __ballot(deg > max(seq, HUB_DEG));
     while (hubs) {
       constexpr int U = 8;
       const int src = __ffsll((unsigned long long)hubs) - 1;

@@ -27,7 +27,7 @@ def near_regular(n, d, wide, seed):
 
 @pytest.mark.parametrize("no_bitmaps", [0, 1])
 @pytest.mark.parametrize("wide", [0, 3])
-@pytest.mark.parametrize("n,d", [(127, 34), (128, 40), (700, 100), (1100, 500), (1300, 520)])
+@pytest.mark.parametrize("n,d", [(127, 34), (128, 40), (700, 100), (700, 128), (900, 256), (1100, 500), (1300, 520)])
 def test_even_lists_expand_the_oracles_nodes(n, d, wide, no_bitmaps):
     g = near_regular(n, d, wide, d)
     G, og = scs.Graph.from_csr(g.off, g.adj), OracleGraph.from_csr(g.n, g.off, g.adj)
