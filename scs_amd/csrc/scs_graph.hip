@@ -201,8 +201,12 @@ __device__ __forceinline__ u64 c_load64(const u64* p) {
 
 // Grid barrier after step `gen`; the last block to arrive decides the next
 // step for all.  scan: the barrier ends a scan that queued `count` vertices,
-// else a peel that finished `count`.  The step comes back in L.
+// else a peel that finished `count`.  The step comes back in L.  Each wave
+// waits for its own operations before the block arrives: the block's barrier
+// alone does not wait for stores and adds that return nothing (a degree's
+// undone decrement, an overflow entry), and other blocks read those next.
 __device__ void core_barrier(CoreCtl* C, CoreLds& L, u32 n, u32 gen, bool scan, u32 count) {
+  c_order();
   __syncthreads();
   if (threadIdx.x == 0) {
     const u32 g = blockIdx.x % CORE_GROUPS, G = gridDim.x;
