@@ -24,8 +24,8 @@
 void scs_pack_model(const scs_model* m, MlpDev* d);
 
 extern "C" {
-int scs_core_run(const i64* off, const int32_t* adj, u32 n, u32* core, u32* tmp,
-                 hipStream_t s);
+int scs_core_run(const i64* off, const int32_t* adj, u32 n, u32* core, u32* tmp, hipStream_t s,
+                 u32 blocks);
 u64 scs_core_words(u32 n);
 hipError_t scs_launch_csr_check(const i64* off, const int32_t* adj, u32 n, u64 nnz, u64* res,
                                 hipStream_t s);
@@ -112,7 +112,7 @@ static int core_decompose(scs_graph* G) {
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
   HIPCHK(hipEventRecord(e0, s));
-  const int rc = scs_core_run(G->d_off, G->d_adj, n, G->d_core, tmp, s);
+  const int rc = scs_core_run(G->d_off, G->d_adj, n, G->d_core, tmp, s, 0);
   HIPCHK(hipEventRecord(e1, s));
   HIPCHK(hipEventSynchronize(e1));
   float ms = 0;

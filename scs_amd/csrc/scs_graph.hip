@@ -117,6 +117,7 @@ extern "C" hipError_t scs_launch_csr_narrow(const i64* off, u32 n, u32* off32, u
 #define CORE_EMPTY 0xffffffffu
 #define CORE_VPB 256        // vertices per block at least
 #define CORE_TIMEOUT 3000000000ull  // wall_clock64 ticks (100 MHz): 30 s
+#define CORE_GRACE 20000ull         // the same, for the blocks to come: 200 us
 
 enum { CORE_SCAN = 0, CORE_PEEL = 1, CORE_OVF = 2, CORE_DONE = 3 };
 
@@ -134,6 +135,8 @@ struct CoreCtl {
   CoreLine grp[CORE_GROUPS];
   CoreLine go[CORE_GROUPS];  // what the group polls: step << 34 | op << 32 | k
   CoreLine root;
+  CoreLine join;  // blocks that have come; high word: closed to others
+  CoreLine nblk;  // blocks that take part (0 while join is open)
   u32 minrest, pad0[31];
   u32 ovf, pad1[31];
   // the root's last block only
@@ -172,6 +175,7 @@ struct CoreLds {
   u32 q[CORE_QCAP];
   u32 head, tail, pending, done;
   u32 found, op, k, o0, o1, mn;
+  u32 rank, nblk;  // this block among those that take part
 };
 __device__ __forceinline__ u32 c_lget(const u32* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -199,6 +203,42 @@ __device__ __forceinline__ u64 c_load64(const u64* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Which blocks take part: those that come before the join closes, which is when
+// the last block of the grid has come, or CORE_GRACE after the first of those
+// still waiting.  A block that comes later leaves at once, so no block ever
+// waits for one that has found no room: on a stream with few CUs, beside
+// another kernel or another peel, the peel runs with the blocks that are there
+// (one is enough).  Their numbers are the block numbers when all have come,
+// else the order of arrival.  False: this block leaves.
+__device__ bool core_join(CoreCtl* C, CoreLds& L) {
+  if (threadIdx.x == 0) {
+    const u32 G = gridDim.x;
+    u32 r = blockIdx.x, nb = 1;
+    if (G > 1) {
+      const u64 old = c_add64(&C->join.v, 1ull);
+      nb = 0;
+      if (!(old >> 32)) {
+        r = (u32)old;
+        const u64 t0 = wall_clock64();
+        while ((nb = (u32)c_load64(&C->nblk.v)) == 0) {
+          if (r + 1 == G || wall_clock64() - t0 > CORE_GRACE) {
+            const u64 o = __hip_atomic_fetch_or(&C->join.v, 1ull << 32, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+            if (!(o >> 32)) c_store64(&C->nblk.v, o);
+          } else {
+            __builtin_amdgcn_s_sleep(1);
+          }
+        }
+        if (nb == G) r = blockIdx.x;
+      }
+    }
+    L.rank = r;
+    L.nblk = nb;
+  }
+  __syncthreads();
+  return L.nblk != 0;
+}
+
 // Grid barrier after step `gen`; the last block to arrive decides the next
 // step for all.  scan: the barrier ends a scan that queued `count` vertices,
 // else a peel that finished `count`.  The step comes back in L.  Each wave
@@ -209,7 +249,7 @@ __device__ void core_barrier(CoreCtl* C, CoreLds& L, u32 n, u32 gen, bool scan, 
   c_order();
   __syncthreads();
   if (threadIdx.x == 0) {
-    const u32 g = blockIdx.x % CORE_GROUPS, G = gridDim.x;
+    const u32 g = L.rank % CORE_GROUPS, G = L.nblk;
     const u32 ingrp = (G - g + CORE_GROUPS - 1) / CORE_GROUPS;
     const u32 ngrp = G < CORE_GROUPS ? G : CORE_GROUPS;
     if (scan && L.mn < c_load(&C->minrest)) atomicMin(&C->minrest, L.mn);
@@ -254,8 +294,8 @@ __device__ void core_barrier(CoreCtl* C, CoreLds& L, u32 n, u32 gen, bool scan, 
         for (u32 i = 0; i < ngrp; i++) c_store64(&C->go[i].v, w);
       }
     }
-    // every block of the grid is resident, so the wait ends; the time limit
-    // only guards against a machine where that does not hold
+    // every block that takes part is running, so the wait ends; the time limit
+    // only guards against a machine that stops some of them
     u64 w;
     const u64 t0 = wall_clock64();
     u32 spins = 0;
@@ -334,7 +374,9 @@ __global__ void __launch_bounds__(CORE_T) core_peel(const i64* __restrict__ off,
                                                     u32 mask, u32* __restrict__ ovf,
                                                     CoreCtl* __restrict__ C) {
   __shared__ CoreLds L;
-  const u32 nt = gridDim.x * CORE_T, tid = blockIdx.x * CORE_T + threadIdx.x;
+  if (!core_join(C, L)) return;
+  const u32 rank = L.rank, nblk = L.nblk;
+  const u32 nt = nblk * CORE_T, tid = rank * CORE_T + threadIdx.x;
   const u32 lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (u32 i = threadIdx.x; i < CORE_QCAP; i += CORE_T) L.q[i] = CORE_EMPTY;
   if (threadIdx.x == 0) {
@@ -389,8 +431,7 @@ __global__ void __launch_bounds__(CORE_T) core_peel(const i64* __restrict__ off,
     u32 done = 0;
     if (op == CORE_OVF) {
       // this block's share of the entries that overflowed, a wave each
-      for (u64 i = (u64)wave * gridDim.x + blockIdx.x; i < o1 - o0;
-           i += (u64)gridDim.x * (CORE_T / 64)) {
+      for (u64 i = (u64)wave * nblk + rank; i < o1 - o0; i += (u64)nblk * (CORE_T / 64)) {
         core_take(off, adj, C, L, ovf, deg, mask, k, c_load(&ovf[o0 + i]));
         done++;
       }
@@ -437,9 +478,8 @@ __global__ void __launch_bounds__(CORE_T) core_peel(const i64* __restrict__ off,
 // ---------------------------------------------------------------------------
 // Host-side launch helpers (C linkage inside the library).
 // ---------------------------------------------------------------------------
-// One block per CU at most (every block must be resident for the grid
-// barrier: 8 waves and 17 KB of LDS), fewer on small graphs, whose levels
-// are too short for every CU to have a share.
+// One block per CU at most (8 waves and 17 KB of LDS), fewer on small graphs,
+// whose levels are too short for every CU to have a share.
 static u32 core_blocks(u32 n) {
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
@@ -459,11 +499,11 @@ static u32 core_pow2(u32 n) {
 extern "C" u64 scs_core_words(u32 n) { return CORE_CTL_WORDS + (1ull << core_pow2(n)) + n; }
 
 // Core numbers of the CSR into core; tmp: scs_core_words(n) words on a
-// 128-byte boundary.  One peel runs on a device at a time: two grids that
-// each wait for all their blocks must not share it.  Waits for the result.
+// 128-byte boundary; blocks: of the grid (0 = as many as suit the graph).
+// Waits for the result.
 static std::mutex g_core_mu;
 extern "C" int scs_core_run(const i64* off, const int32_t* adj, u32 n, u32* core, u32* tmp,
-                            hipStream_t s) {
+                            hipStream_t s, u32 blocks) {
   if (n == 0) return SCS_OK;
   std::lock_guard<std::mutex> lk(g_core_mu);
   CoreCtl* C = (CoreCtl*)tmp;
@@ -473,7 +513,7 @@ extern "C" int scs_core_run(const i64* off, const int32_t* adj, u32 n, u32* core
   const u32 ib = (n + 255) / 256;
   core_init<<<ib < 4096 ? ib : 4096, 256, 0, s>>>(off, n, deg, (u32)(slots - 1), C);
   if (hipGetLastError() != hipSuccess) return SCS_EHIP;
-  core_peel<<<core_blocks(n), CORE_T, 0, s>>>(off, adj, n, core, deg, (u32)(slots - 1), ovf, C);
+  core_peel<<<blocks ? blocks : core_blocks(n), CORE_T, 0, s>>>(off, adj, n, core, deg, (u32)(slots - 1), ovf, C);
   if (hipGetLastError() != hipSuccess) return SCS_EHIP;
   u32 failed = 0;
   if (hipMemcpyAsync(&failed, &C->failed, sizeof(u32), hipMemcpyDeviceToHost, s) != hipSuccess ||
@@ -517,5 +557,5 @@ extern "C" int scs_core_numbers_noalloc(const int64_t* d_off, const int32_t* d_a
   u32* S = nullptr;
   const int rc = scratch_address(&S);
   if (rc) return rc;
-  return scs_core_run(d_off, d_adj, n, d_core, S, (hipStream_t)stream);
+  return scs_core_run(d_off, d_adj, n, d_core, S, (hipStream_t)stream, 0);
 }
