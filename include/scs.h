@@ -161,7 +161,7 @@ double scs_graph_core_time_us(const scs_graph* g);
  * GPU, held until the process ends), so n is at most 2^20 (SCS_EBIG beyond).
  * Allocates nothing.  Waits for the result (so it cannot be captured into a
  * graph).  Every call on one GPU uses that GPU's array: calls of one process
- * take turns, calls of several threads included.  The kernel runs
+ * on that GPU take turns, calls of several threads included.  The kernel runs
  * with the blocks that find room (8 waves and 17 KB of LDS each), so it also
  * works on a stream confined to few CUs; beside a search epoch that holds the
  * LDS of every CU it starts when the epoch ends. */

@@ -499,13 +499,11 @@ static u32 core_pow2(u32 n) {
 extern "C" u64 scs_core_words(u32 n) { return CORE_CTL_WORDS + (1ull << core_pow2(n)) + n; }
 
 // Core numbers of the CSR into core; tmp: scs_core_words(n) words on a
-// 128-byte boundary; blocks: of the grid (0 = as many as suit the graph).
-// Waits for the result.
-static std::mutex g_core_mu;
+// 128-byte boundary, this call's own; blocks: of the grid (0 = as many as suit
+// the graph).  Waits for the result.
 extern "C" int scs_core_run(const i64* off, const int32_t* adj, u32 n, u32* core, u32* tmp,
                             hipStream_t s, u32 blocks) {
   if (n == 0) return SCS_OK;
-  std::lock_guard<std::mutex> lk(g_core_mu);
   CoreCtl* C = (CoreCtl*)tmp;
   const u64 slots = 1ull << core_pow2(n);
   u32* deg = tmp + CORE_CTL_WORDS;
@@ -533,29 +531,26 @@ extern "C" int scs_core_run(const i64* off, const int32_t* adj, u32 n, u32* core
 static __device__ __align__(256) u32 scratch[CORE_CTL_WORDS + 2u * CORE_NA_MAX_N];
 
 #define CORE_NA_DEVICES 64
-static u32* g_scratch_dev[CORE_NA_DEVICES];
-static std::mutex g_scratch_mu;
-
-static int scratch_address(u32** out) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= CORE_NA_DEVICES) return SCS_EHIP;
-  std::lock_guard<std::mutex> lk(g_scratch_mu);
-  if (!g_scratch_dev[dev]) {
-    void* p = nullptr;
-    if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p) return SCS_EHIP;
-    g_scratch_dev[dev] = (u32*)p;
-  }
-  *out = g_scratch_dev[dev];
-  return SCS_OK;
-}
+// The array of each device; its lock is held for a call, so calls on one
+// device take turns and those on others do not wait for them.
+static struct CoreScratch {
+  std::mutex mu;
+  u32* words = nullptr;
+} g_scratch[CORE_NA_DEVICES];
 
 extern "C" int scs_core_numbers_noalloc(const int64_t* d_off, const int32_t* d_adj, uint32_t n,
                                         uint32_t* d_core, void* stream) {
   if (!d_off || !d_core || (n && !d_adj)) return SCS_EINVAL;
   if (n > CORE_NA_MAX_N) return SCS_EBIG;
   if (n == 0) return SCS_OK;
-  u32* S = nullptr;
-  const int rc = scratch_address(&S);
-  if (rc) return rc;
-  return scs_core_run(d_off, d_adj, n, d_core, S, (hipStream_t)stream, 0);
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= CORE_NA_DEVICES) return SCS_EHIP;
+  CoreScratch& S = g_scratch[dev];
+  std::lock_guard<std::mutex> lk(S.mu);
+  if (!S.words) {
+    void* p = nullptr;
+    if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p) return SCS_EHIP;
+    S.words = (u32*)p;
+  }
+  return scs_core_run(d_off, d_adj, n, d_core, S.words, (hipStream_t)stream, 0);
 }

@@ -1,7 +1,9 @@
 """Core numbers on a GPU that is not the call's alone: more blocks than find room
-(those that come late take no part)."""
+(those that come late take no part), and calls that do not wait for each other
+where they share nothing."""
 
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -42,6 +44,12 @@ class Peel:
             b.free()
 
 
+def _stream(hip):
+    s = C.c_void_p()
+    assert hip.hipStreamCreateWithFlags(C.byref(s), 1) == 0  # not blocked by the default stream
+    return s
+
+
 @pytest.mark.parametrize("blocks", [1, 2, 9, 300, 4096])
 def test_any_number_of_blocks(blocks):
     """4,096 blocks of 512 threads are more than the GPU holds at once (at most
@@ -53,3 +61,57 @@ def test_any_number_of_blocks(blocks):
         p.run(blocks=blocks)
         p.check()
     p.close()
+
+
+def test_peels_of_several_streams_at_once():
+    hip = _hip()
+    peels = [Peel(hip, 30000, 10 + i, i) for i in range(4)]
+    streams = [_stream(hip) for _ in peels]
+    print("4 peels at once", flush=True)
+    errors = []
+
+    def work(p, s):
+        try:
+            for _ in range(3):
+                p.run(s)
+        except AssertionError as e:
+            errors.append(e)
+
+    ts = [threading.Thread(target=work, args=a) for a in zip(peels, streams)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not errors
+    for p, s in zip(peels, streams):
+        p.check()
+        hip.hipStreamDestroy(s)
+        p.close()
+
+
+def test_a_call_does_not_wait_for_another_stream():
+    """A call whose stream still waits for the host holds up no call on another
+    stream."""
+    hip = _hip()
+    a, b = Peel(hip, 5000, 8, 1), Peel(hip, 5000, 8, 2)
+    sa, sb = _stream(hip), _stream(hip)
+    go = threading.Event()
+    done_a, done_b = threading.Event(), threading.Event()
+    wait = C.CFUNCTYPE(None, C.c_void_p)(lambda _: go.wait(20))
+    assert hip.hipLaunchHostFunc(sa, wait, None) == 0
+    ta = threading.Thread(target=lambda: (a.run(sa), done_a.set()))
+    tb = threading.Thread(target=lambda: (b.run(sb), done_b.set()))
+    ta.start()
+    tb.start()
+    print("one stream held by the host", flush=True)
+    free = done_b.wait(5) and not done_a.is_set()
+    go.set()
+    ta.join()
+    tb.join()
+    assert free
+    a.check()
+    b.check()
+    for s in (sa, sb):
+        hip.hipStreamDestroy(s)
+    a.close()
+    b.close()
