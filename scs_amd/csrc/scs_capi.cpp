@@ -59,6 +59,7 @@ hipError_t scs_launch_ms_scan_loff(u32 nb, const MsBatch* B, u32* tot, u64 valid
 hipError_t scs_launch_ms_fill(const int32_t* adj, const MsUnit* units, u32 nunits,
                               const u64* vis, u64 valid, u64 packed, const u32* locid,
                               const MsBatch* B, const u32* hubcnt, unsigned long long* bytes, hipStream_t s);
+u32 scs_epoch_lds_spare(u32 waves_per_cu, u32 n);
 hipError_t scs_launch_epoch(const EngineArgs* A, hipStream_t s);
 hipError_t scs_launch_slot_write(const QuerySlot* stage, const u32* idx, const u32* wit, u32 n,
                                  QuerySlot* slots, u32* witness, hipStream_t s);
@@ -720,6 +721,7 @@ extern "C" int scs_engine_create(scs_graph* g, const scs_params* pin, scs_engine
     const u32 fit = (u32)std::min<u64>(w, (16ull << 30) / (lay.zstride + lay.gstride));
     if (E->heu_gpu.init(g->hg.n, w, std::max<u32>(fit, 16), SCS_MAX_H) != SCS_OK)
       return fail(SCS_ENOMEM);
+    A.lds_spare = scs_epoch_lds_spare(A.waves_per_cu, n);
   }
   E->st.waves = E->nwaves;
   E->st.kcap = E->kcap;

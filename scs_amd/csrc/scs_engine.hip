@@ -111,8 +111,8 @@ struct Lds {
   u64 tph[SCS_PHASES];      // wall-clock ticks per phase (lane 0 adds)
   u32 D[SCS_FRAME_DOMS];
   u32 hist[SCS_HCAP + 4];   // dC histogram of R (live copy of the wave's state)
-  u64 tot[64];              // per-vertex sums of a scan_adj step
   union __attribute__((aligned(8))) {  // never live at the same time within a node
+    u64 tot[64];              // per-vertex sums of a scan_adj step
     u32 chist[SCS_HCAP + 4];  // scratch histogram of C degrees (U_nr)
     u16 h1s[16 * MLP_H];      // MLP hidden-layer tile (bf16), 8-byte aligned
   };
@@ -2419,19 +2419,34 @@ __global__ void __launch_bounds__(64, 2) __attribute__((flatten)) scs_epoch(Engi
 }
 
 // Dynamic LDS of one wave: its share of the CU's 160 KB at the requested
-// waves per CU, minus the static part, capped at 48 KB.  2 KB per CU stay free
-// for the heuristic's blocks, which run beside an epoch.
-static u32 epoch_lds_bytes(u32 waves_per_cu) {
+// waves per CU, minus the static part, capped at 48 KB.  The CU hands its LDS
+// out in 128 pieces of 1,280 bytes, so the share is counted in those (a share
+// of 158 KB / 4 takes as many pieces as one of 160 KB / 4); `spare` pieces per
+// CU stay free.
+#define LDS_PIECES 128u
+#define LDS_PIECE 1280u
+extern "C" u32 scs_epoch_lds_bytes(u32 waves_per_cu, u32 spare) {
   const u32 wpc = waves_per_cu ? waves_per_cu : 16;
-  const i64 share = (i64)(158 * 1024 / wpc) - (i64)sizeof(Lds);
-  i64 b = share < (i64)(48 * 1024) ? share : (i64)(48 * 1024);
-  b = b > 0 ? (b & ~(i64)511) : 0;
-  return (u32)b;
+  const i64 share = (i64)((LDS_PIECES - spare) / wpc * LDS_PIECE) - (i64)sizeof(Lds);
+  const i64 b = share < (i64)(48 * 1024) ? share : (i64)(48 * 1024);
+  return b > 0 ? (u32)(b & ~(i64)7) : 0u;
+}
+// Pieces to leave free for the heuristic's blocks (one each), so that they run
+// beside an epoch instead of after it: on 4,000 vertices four queries' bounds
+// come after 1 ms, 201 ms (the epoch's time slice) without.  With more than
+// one search wave per SIMD no block finds registers, and where the graph's
+// bitmaps fit the full share and not the smaller one, the search needs it more.
+extern "C" u32 scs_epoch_lds_spare(u32 waves_per_cu, u32 n) {
+  if (waves_per_cu > 4) return 0;
+  const u32 need = 8 * ((n + 31) / 32);
+  const bool lost = need <= scs_epoch_lds_bytes(waves_per_cu, 0) &&
+                    need > scs_epoch_lds_bytes(waves_per_cu, 1);
+  return lost ? 0 : 1;
 }
 
 extern "C" hipError_t scs_launch_epoch(const EngineArgs* A, hipStream_t s) {
   EngineArgs a = *A;
-  const u32 dyn = epoch_lds_bytes(a.waves_per_cu);
+  const u32 dyn = scs_epoch_lds_bytes(a.waves_per_cu, a.lds_spare);
   a.lds_words = a.no_bitmaps ? 0u : dyn / 4;
   if (a.model)
     scs_epoch<true><<<a.nwaves, 64, dyn, s>>>(a);
