@@ -309,10 +309,26 @@ struct HeuGpu {
   u32* d_H3 = nullptr;    // 3 * waves * SCS_MAX_H
   std::vector<u32> h_out, h_H;
 
-  // room for `fit` queries of h <= hmax at once (more of smaller h)
+  // Queries of h <= hmax at once: `w` within 16 GiB of workspace (a launch lasts
+  // as long as its slowest query), but `least` of them.
+  static u32 fit_for(u32 n, u32 w, u32 least, u32 hmax) {
+    const HeuLayout lay = scs_heu_layout(n, hmax);
+    const u64 f = (16ull << 30) / (lay.zstride + lay.gstride);
+    return std::min(w, (u32)std::min<u64>(std::max<u64>(f, least), w));
+  }
+  // Calls of up to `w` queries, with room for `fit` of h <= hmax per launch (more
+  // of smaller h), or for half of that, and so on, where the memory is not there.
   int init(u32 n_, u32 w, u32 fit, u32 hmax) {
     n = n_;
     waves = w;
+    while (true) {
+      const int rc = alloc(fit, hmax);
+      if (rc != SCS_ENOMEM) return rc;
+      if (fit == 1) return SCS_EHIP;
+      fit /= 2;
+    }
+  }
+  int alloc(u32 fit, u32 hmax) {
     const HeuLayout lay = scs_heu_layout(n, hmax);
     zbytes = lay.zstride * fit;
     gbytes = lay.gstride * fit;
@@ -329,7 +345,11 @@ struct HeuGpu {
       at[i] = o;
       o += (part[i] + 255) & ~255ull;
     }
-    HIPCHK(hipMalloc(&zs, o));
+    if (hipMalloc(&zs, o) != hipSuccess) {
+      (void)hipGetLastError();  // not for the next launch to report
+      zs = nullptr;
+      return SCS_ENOMEM;
+    }
     HIPCHK(hipMemset(zs, 0, zbytes));
     gs = zs + at[1];
     d_in = (u32*)(zs + at[2]);
@@ -391,7 +411,7 @@ extern "C" int scs_heuristic_gpu(const scs_graph* g, uint32_t count, const uint3
   u32 hmax = 1;
   for (u32 i = 0; i < count; i++) hmax = std::max(hmax, h[i]);
   const u32 w = std::min<u32>(count, 64);
-  int rc = hg.init(g->hg.n, w, w, hmax);
+  int rc = hg.init(g->hg.n, w, HeuGpu::fit_for(g->hg.n, w, 1, hmax), hmax);
   hipStream_t s = nullptr;
   if (rc == SCS_OK && hipStreamCreate(&s) != hipSuccess) rc = SCS_EHIP;
   std::vector<std::vector<u32>> HH(hg.waves);
@@ -714,12 +734,9 @@ extern "C" int scs_engine_create(scs_graph* g, const scs_params* pin, scs_engine
   E->h_slots.resize(nq);
   E->heu_work.resize(p.heuristic_threads);
   if (p.gpu_heuristic && g->d_off32) {
-    // as many queries per launch as an admission step takes, within 16 GiB
-    // of workspace (a launch lasts as long as its slowest query)
-    const HeuLayout lay = scs_heu_layout(g->hg.n, SCS_MAX_H);
+    // as many queries per launch as an admission step takes
     const u32 w = std::max<u32>(p.admit_per_step, 64);
-    const u32 fit = (u32)std::min<u64>(w, (16ull << 30) / (lay.zstride + lay.gstride));
-    if (E->heu_gpu.init(g->hg.n, w, std::max<u32>(fit, 16), SCS_MAX_H) != SCS_OK)
+    if (E->heu_gpu.init(n, w, HeuGpu::fit_for(n, w, 7, SCS_MAX_H), SCS_MAX_H) != SCS_OK)
       return fail(SCS_ENOMEM);
     A.lds_spare = scs_epoch_lds_spare(A.waves_per_cu, n);
   }
