@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <chrono>
 #include <cstdio>
@@ -565,6 +566,25 @@ static WaveLayout make_layout(u32 kcap) {
   return L;
 }
 
+// The batched preprocessing's buffers of a graph of n vertices: bytes of each,
+// in the order of PREP_BUFS.
+enum { PREP_MASKS = 5, PREP_DIST = 5, PREP_LOCID, PREP_GCNT, PREP_CBASE, PREP_BUFS };
+static std::array<u64, PREP_BUFS> prep_buffers(u32 n) {
+  const u64 n1 = std::max<u32>(n, 1), G = (n1 + 63) / 64;
+  std::array<u64, PREP_BUFS> b;
+  for (u32 i = 0; i < PREP_MASKS; i++) b[i] = sizeof(u64) * n1;
+  b[PREP_DIST] = sizeof(u16) * 64 * n1;
+  b[PREP_LOCID] = sizeof(u32) * 64 * n1;
+  b[PREP_GCNT] = sizeof(u32) * 64 * G;
+  b[PREP_CBASE] = sizeof(u32) * 64 * scs_ms_count_rows((u32)G);
+  return b;
+}
+extern "C" u64 scs_prep_buffer_bytes(u32 n) {
+  u64 sum = 0;
+  for (u64 b : prep_buffers(n)) sum += b;
+  return sum;
+}
+
 extern "C" int scs_engine_create(scs_graph* g, const scs_params* pin, scs_engine** out) {
   if (!g || !out) return SCS_EINVAL;
   scs_params p;
@@ -605,7 +625,7 @@ extern "C" int scs_engine_create(scs_graph* g, const scs_params* pin, scs_engine
     // preprocessing buffers; larger kept sets are rejected per query
     size_t freeb = 0, totalb = 0;
     if (hipMemGetInfo(&freeb, &totalb) != hipSuccess) return fail(SCS_EHIP);
-    const u64 fixed = p.mem_budget + 420ull * n + (64ull << 20);
+    const u64 fixed = p.mem_budget + scs_prep_buffer_bytes(n) + (64ull << 20);
     const u64 room = freeb > fixed ? (u64)((freeb - fixed) * 0.6) : 0;
     const u64 pool_slots = std::max<u64>(p.limit_tasks ? p.limit_tasks : 2ull * E->nwaves,
                                          (u64)E->nwaves + p.limit_queries + 64);
@@ -636,14 +656,14 @@ extern "C" int scs_engine_create(scs_graph* g, const scs_params* pin, scs_engine
   if (hipMalloc(&E->d_pool_pos, sizeof(u64) * 2) != hipSuccess) return fail(SCS_ENOMEM);
   if (hipMalloc(&E->d_glob, sizeof(EngineGlobals)) != hipSuccess) return fail(SCS_ENOMEM);
   const u32 n1 = std::max<u32>(n, 1);
-  const u64 G = (n1 + 63) / 64;
-  for (u64** b : {&E->d_elig, &E->d_vis, &E->d_fr, &E->d_nf, &E->d_xf})
-    if (hipMalloc(b, sizeof(u64) * n1) != hipSuccess) return fail(SCS_ENOMEM);
-  if (hipMalloc(&E->d_dist16, sizeof(u16) * 64 * (u64)n1) != hipSuccess) return fail(SCS_ENOMEM);
-  if (hipMalloc(&E->d_locid64, sizeof(u32) * 64 * (u64)n1) != hipSuccess) return fail(SCS_ENOMEM);
-  if (hipMalloc(&E->d_gcnt, sizeof(u32) * 64 * G) != hipSuccess) return fail(SCS_ENOMEM);
-  if (hipMalloc(&E->d_cbase, sizeof(u32) * 64 * scs_ms_count_rows((u32)G)) != hipSuccess)
-    return fail(SCS_ENOMEM);
+  {
+    const std::array<u64, PREP_BUFS> bytes = prep_buffers(n);
+    void** const at[PREP_BUFS] = {(void**)&E->d_elig,   (void**)&E->d_vis,     (void**)&E->d_fr,
+                                  (void**)&E->d_nf,     (void**)&E->d_xf,      (void**)&E->d_dist16,
+                                  (void**)&E->d_locid64, (void**)&E->d_gcnt,   (void**)&E->d_cbase};
+    for (u32 i = 0; i < PREP_BUFS; i++)
+      if (hipMalloc(at[i], bytes[i]) != hipSuccess) return fail(SCS_ENOMEM);
+  }
   {
     // adjacency units: one per vertex, or ceil(deg / MS_UNIT) for a hub
     std::vector<MsUnit> units;
