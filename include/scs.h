@@ -72,7 +72,8 @@ typedef struct scs_params {
   uint32_t buffer_size;    /* argv[3]: words of the shared task pool
                               (0 = derived from limit_tasks) */
   double copy_limit;       /* argv[4]: a wave donates work while fewer than
-                              copy_limit * waves tasks are pooled */
+                              copy_limit * waves tasks are pooled, and fewer than
+                              there are idle waves */
   uint32_t read_limit;     /* argv[5]: kept for the command line; one task is
                               taken per visit to the pool */
   uint32_t limit_queries;  /* argv[6]: resident query slots */
