@@ -120,7 +120,8 @@ typedef struct scs_params {
                               counts and witness in every mode */
   uint32_t gpu_heuristic;  /* 1 = admission computes CSSC_heu (inc/heuristic.h:321-348) on
                               the GPU, three blocks per query, instead of on host threads;
-                              same kl and H (needs fewer than 2^32 adjacency entries) */
+                              same kl and H (needs fewer than 2^32 - 4096 adjacency
+                              entries) */
 } scs_params;
 
 typedef struct scs_result {
@@ -228,7 +229,7 @@ int scs_heuristic_csr(const int64_t* off, const int32_t* adj, uint32_t n, uint32
 /* The same greedy lower bound (inc/heuristic.h:8-348) for `count` queries on
  * the GPU, one block per construction of each query, on a resident graph: kl[i], hsize[i] (the size
  * of H, also when it exceeds cap) and H row i (up to cap ids).  Equal to
- * scs_heuristic_csr value for value.  SCS_EBIG when the graph has 2^32
+ * scs_heuristic_csr value for value.  SCS_EBIG when the graph has 2^32 - 4096
  * adjacency entries or more. */
 int scs_heuristic_gpu(const scs_graph* g, uint32_t count, const uint32_t* l,
                       const uint32_t* h, const uint32_t* q, uint32_t* kl, uint32_t* hsize,

@@ -99,7 +99,7 @@ struct scs_graph {
   u32* d_core = nullptr;
   // the search's view of the whole graph (queries that keep most of it
   // search it in place): 32-bit offsets and the identity id map; null when
-  // the adjacency has 2^32 entries or more
+  // the adjacency is too long for them (scs_csr_fits32)
   u32* d_off32 = nullptr;
   u32* d_ident = nullptr;
   double core_us = 0;
@@ -129,6 +129,12 @@ static int core_decompose(scs_graph* G) {
   return rc;
 }
 
+// Whether the search and the heuristic may read the resident CSR through 32-bit
+// offsets.  Their loops run up to a row's end in steps of at most 2,048 entries
+// and compare an index up to two steps past it, which must not wrap: with a row
+// that ends within 2,048 entries of 2^32 the heuristic's loops would not end.
+extern "C" int scs_csr_fits32(u64 nnz) { return nnz < (1ull << 32) - 4096; }
+
 // The CSR to the device, and what the host keeps of it.  check: the rows come
 // from a caller and are validated on the device before any other kernel reads
 // them; the host copies its own while that runs.
@@ -144,7 +150,7 @@ static int graph_upload(scs_graph* G, const int64_t* off, const int32_t* adj, u3
     HIPCHK(hipMemset(res, 0, 3 * sizeof(u64)));
     HIPCHK(scs_launch_csr_check(G->d_off, G->d_adj, n, nnz, res, nullptr));
   }
-  if (nnz <= 0xffffffffull) {
+  if (scs_csr_fits32(nnz)) {
     HIPCHK(hipMalloc(&G->d_off32, sizeof(u32) * (n + 1ull)));
     HIPCHK(hipMalloc(&G->d_ident, sizeof(u32) * std::max<u64>(n, 1)));
     HIPCHK(scs_launch_csr_narrow(G->d_off, n, G->d_off32, G->d_ident, nullptr));
