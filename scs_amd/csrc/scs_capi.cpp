@@ -69,7 +69,7 @@ hipError_t scs_launch_admit(const EngineArgs* A, const u32* slots, u32 n, u32* f
                             hipStream_t s);
 hipError_t scs_launch_pool_init(u64* seq, u32 n, hipStream_t s);
 HeuLayout scs_heu_layout(u32 n, u32 hmax);
-hipError_t scs_launch_heu(const u32* off, const u32* adj, u32 n, u32 dmax, u32 nq, const u32* ql,
+hipError_t scs_launch_heu(const u32* off, const u32* adj, u32 dmax, u32 nq, const u32* ql,
                           const u32* qh, const u32* qq, u8* zs, u8* gs, HeuLayout lay, u32 hcap, u32* kl,
                           u32* hsize, u32* H, u32* kl3, u32* hs3, u32* H3, hipStream_t s);
 }
@@ -389,7 +389,7 @@ struct HeuGpu {
     if (fit == 0) return SCS_ENOMEM;
     HIPCHK(hipMemcpyAsync(d_in, in.data(), sizeof(u32) * 3 * cnt, hipMemcpyHostToDevice, s));
     for (u32 i0 = 0; i0 < cnt; i0 += fit)
-      HIPCHK(scs_launch_heu(g->d_off32, (const u32*)g->d_adj, n, g->hg.dmax,
+      HIPCHK(scs_launch_heu(g->d_off32, (const u32*)g->d_adj, g->hg.dmax,
                             std::min(fit, cnt - i0), d_in + i0, d_in + cnt + i0,
                             d_in + 2 * cnt + i0, zs, gs, lay, SCS_MAX_H, d_out + i0, d_out + cnt + i0,
                             d_H + (u64)i0 * SCS_MAX_H, d_out3, d_out3 + 3 * waves, d_H3, s));

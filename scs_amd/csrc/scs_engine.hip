@@ -106,7 +106,7 @@ __device__ __forceinline__ u32 ubd_node(u32 kl, u32 h) {
 
 // LDS of one wave (one workgroup).
 struct Lds {
-  u32 cnt, cnt2, nfront, ncand, nh, nk, pad0, pad1;
+  u32 cnt, cnt2, nfront, ncand, nk;
   u32 root[8];              // payload of a level root this wave starts itself
   u64 tph[SCS_PHASES];      // wall-clock ticks per phase (lane 0 adds)
   u32 D[SCS_FRAME_DOMS];
@@ -290,12 +290,12 @@ __device__ __forceinline__ void build_bitmaps(W& w) {
 // follow the degrees, take 615 ms with 128 and 256; 618 to 650 with 512 and
 // 512, 725 without even lists, 645 with 96 and 96, 603 with 96 and 512.
 //
-// A level root's neighbour count on a 50,000-vertex, 750,000-edge power-law
-// graph takes 3.4 ms, 16 ms with one 64-entry chunk of one vertex at a time.
-// With the loops over R and the trail taking 4 to 8 vertices per lane at once
-// and the shared words polled without fences, a batch of 64 queries of that
-// graph (16 nodes each) went from 1,236 to 177 ms, and a 64-query
-// batch of proofs on 20,000 vertices from 243 to 44 ms.
+// These scans, loops over R and the trail that take 4 to 8 vertices per lane at
+// once, shared words polled without fences, grown level roots (grow_root) and
+// the closure's choice (r12) together: those eight batches take 585 to 600 ms,
+// 7,500 to 7,860 with one list per lane up to 32 entries, one 64-entry chunk at
+// a time beyond and none of the rest; eight batches of 64 proofs on 20,000
+// vertices 204 ms, 1,060 to 1,070.
 // ---------------------------------------------------------------------------
 #define SEQ_DEG 32u
 #define HUB_DEG 128u

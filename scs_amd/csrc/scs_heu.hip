@@ -47,7 +47,7 @@
 struct HeuArgs {
   const u32* off;  // n+1, 32-bit offsets of the resident graph
   const u32* adj;
-  u32 n, dmax, nq, hcap;
+  u32 dmax, nq, hcap;
   const u32* ql;
   const u32* qh;
   const u32* qq;
@@ -71,7 +71,8 @@ struct __attribute__((aligned(16))) HV {
   u32 cnt, deg, pos, sta;
 };
 
-// The little LDS a block uses leaves it room beside the search kernel.
+// One 1,280-byte piece of the CU's LDS, which an engine that admits through this
+// kernel leaves free beside its search waves.
 struct HL {
   u64 wmax[HEU_NW];
   u32 wmin[HEU_NW];
@@ -79,7 +80,7 @@ struct HL {
   u32 dv[2];    // H-neighbours of the chosen vertex (by step parity)
   u32 rank[2];  // members of H with a smaller id (by step parity)
   u32 best[2];  // heu3: largest id + 1 among the equal keys (by step parity)
-  u32 step, mindeg, remove;
+  u32 mindeg, remove;
   u64 bk[HEU_LDSB];
 };
 
@@ -104,7 +105,7 @@ __device__ __forceinline__ u64 h_below() { return LANE ? (~0ull >> (64 - LANE)) 
 struct HW {
   const u32* off;
   const u32* adj;
-  u32 n, dmax, W;
+  u32 dmax, W;
   HV* hv;
   u64* key;   // heu3: bits of the largest score pushed, plus one
   u64* mask;  // heu3: W words per vertex, bit j = adjacent to the j-th member of H
@@ -680,7 +681,6 @@ __global__ void __launch_bounds__(HEU_T, 4) scs_heu_kernel(HeuArgs A) {
   HW w;
   w.off = A.off;
   w.adj = A.adj;
-  w.n = A.n;
   w.dmax = A.dmax;
   w.W = A.lay.words;
   w.hv = (HV*)z;
@@ -757,14 +757,13 @@ extern "C" HeuLayout scs_heu_layout(u32 n, u32 hmax) {
 
 // zs and gs hold nq workspaces; kl3/hs3/H3 hold the three constructions'
 // results of each query, kl/hsize/H the picked one.
-extern "C" hipError_t scs_launch_heu(const u32* off, const u32* adj, u32 n, u32 dmax, u32 nq,
+extern "C" hipError_t scs_launch_heu(const u32* off, const u32* adj, u32 dmax, u32 nq,
                                      const u32* ql, const u32* qh, const u32* qq, u8* zs,
                                      u8* gs, HeuLayout lay, u32 hcap, u32* kl, u32* hsize, u32* H,
                                      u32* kl3, u32* hs3, u32* H3, hipStream_t s) {
   HeuArgs A;
   A.off = off;
   A.adj = adj;
-  A.n = n;
   A.dmax = dmax;
   A.nq = nq;
   A.hcap = hcap;

@@ -1,8 +1,9 @@
 // Training and stand-alone inference kernels of the branching MLP.
 //
-// Training runs in FP32 on the vector ALUs (forward, backward, weight
-// gradients, Adam), one launch sequence per mini-batch; inference uses the
-// same BF16 MFMA tile routine as the search engine (scs_mlp.h).
+// Training runs in FP32: a mini-batch is one kernel for the forward and
+// backward pass and the weight gradients, on the FP32 matrix units, and one for
+// their sum and the Adam step.  Inference uses the same BF16 MFMA tile routine
+// as the search engine (scs_mlp.h).
 #include <hip/hip_runtime.h>
 
 #include <cmath>

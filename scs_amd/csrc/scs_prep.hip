@@ -345,7 +345,7 @@ __global__ void __launch_bounds__(256) ms_count(u32 n, u32 G, u32 ch, u64* __res
 // Chunk counts -> exclusive bases in place; K_b -> tot[b].  One wave, lane =
 // query, eight coalesced rows in flight.  (One wave per query over the
 // group counts, 256 bytes apart per lane, took 62 us on 500,000 vertices;
-// counting by chunks first leaves 245 rows.)
+// counting by chunks first leaves 253 rows.)
 __global__ void __launch_bounds__(64) ms_bscan(u32 C, u32* __restrict__ cbase,
                                                u32* __restrict__ tot, unsigned long long* bytes) {
   const u32 b = threadIdx.x;
